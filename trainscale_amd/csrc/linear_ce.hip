@@ -88,8 +88,10 @@ struct GemmArgs {
   int64_t M, N, K;
   __bf16* C;      // bf16 output (modes 0, 1, 4, 6, 7; optional in 5)
   int64_t ldc;
-  float* C32;     // fp32 accumulator (modes 2, 3, 4)
+  float* C32;     // fp32 accumulator (modes 2, 3, 4); one [M, ldc32] slot per K split
   int64_t ldc32;
+  int64_t splits;  // K slots (ts_plan::hidden_split), 0 or 1: K in one piece
+  int64_t kper;    // k per slot
   // logits epilogue
   float2* stats;          // [M][2 * NT] (max, sum exp) per 128-column slice
   // statistics / dlogits epilogues (kEpiStats, kEpiDlogits)
@@ -133,8 +135,10 @@ __device__ inline void stage_f32_tile(const Acc<kTI>& acc, int i, uint8_t* regio
 }
 
 // One 256 x 256 tile of C = A B^T with kW waves (ts_gemm::Cfg) and the
-// epilogue of kMode: tile number `bid` of the GEMM (ts_plan::gemm_tile_of
-// maps it to a tile), `smem` the workgroup's kLdsBytes of LDS.
+// epilogue of kMode: piece number `bid` of the GEMM (ts_plan::gemm_piece_of
+// maps it to a K slot and a tile), `smem` the workgroup's kLdsBytes of LDS.
+// Only the fp32 modes kEpiF32 and kEpiAccF32 take more than one K slot: slot s
+// has its own C32.
 template <int kMode, int kMA, int kMB, int kW>
 __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) {
   using Cw = ts_gemm::Cfg<kW>;
@@ -142,11 +146,32 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
   const int64_t MT = (a.M + BM - 1) / BM;
   const int64_t NT = (a.N + BN - 1) / BN;
   int64_t mt, nt;
-  ts_plan::gemm_tile_of(bid, MT, NT, mt, nt);
+  const __bf16* A = a.A;
+  const __bf16* B = a.B;
+  float* C32 = a.C32;
+  int64_t K = a.K;
+  if constexpr (kMode == kEpiF32 || kMode == kEpiAccF32) {
+    int64_t slot;
+    ts_plan::gemm_piece_of(bid, MT, NT, a.splits > 1 ? a.splits : 1, slot, mt, nt);
+    if (a.splits > 1) {
+      const int64_t k0 = slot * a.kper;
+      K = K - k0 < a.kper ? K - k0 : a.kper;
+      if (K <= 0) {  // uniform: a last chunk shorter than the slots
+        if constexpr (kMode == kEpiAccF32) return;
+        K = 0;       // kEpiF32 writes zeros
+      }
+      const int64_t ks = K > 0 ? k0 : 0;
+      A += kMA == ts_gemm::kKMajor ? ks : ks * a.lda;
+      B += kMB == ts_gemm::kKMajor ? ks : ks * a.ldb;
+      C32 += slot * a.M * a.ldc32;
+    }
+  } else {
+    ts_plan::gemm_tile_of(bid, MT, NT, mt, nt);
+  }
   const int64_t m0 = mt * BM;
   const int64_t n0 = nt * BN;
   Acc<kTI> acc;
-  ts_gemm::mainloop<kMA, kMB, kW>(a.A, a.lda, a.M, a.B, a.ldb, a.N, a.K, m0, n0, smem, acc);
+  ts_gemm::mainloop<kMA, kMB, kW>(A, a.lda, a.M, B, a.ldb, a.N, K, m0, n0, smem, acc);
 
   const int wid = threadIdx.x >> 6;
   const int lane = threadIdx.x & 63;
@@ -225,7 +250,7 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
           for (int q = 0; q < kPre; ++q) {
             const int64_t gm = gm0 + 2 * (h + q);
             const bool in = gm < a.M && gc < a.N;  // N % 8 == 0: 4 columns all in or all out
-            old[q] = in ? *reinterpret_cast<const float4*>(a.C32 + gm * a.ldc32 + gc)
+            old[q] = in ? *reinterpret_cast<const float4*>(C32 + gm * a.ldc32 + gc)
                         : make_float4(0.f, 0.f, 0.f, 0.f);
           }
         }
@@ -252,7 +277,7 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
               pk.y = __builtin_bit_cast(uint32_t, hi);
               *reinterpret_cast<uint2*>(a.C + gm * a.ldc + gc) = pk;
             } else {
-              *reinterpret_cast<float4*>(a.C32 + gm * a.ldc32 + gc) = v;
+              *reinterpret_cast<float4*>(C32 + gm * a.ldc32 + gc) = v;
             }
           }
         }
@@ -687,6 +712,35 @@ __global__ __launch_bounds__(256) void flce_dlogits_kept(__bf16* __restrict__ L,
   st16_stream(p, Elt<__bf16>::pack(g));
 }
 
+// grad_hidden from the K slots of a split GEMM (ts_plan::hidden_split): the slots'
+// fp32 partials [slots][n] added in slot order and rounded once to bf16. A thread
+// owns 4 consecutive elements (n % 4 == 0: rows of H % 8 == 0 elements) and keeps
+// kSumUnroll slots' 16-byte loads in flight.
+constexpr int kSumUnroll = 8;
+__global__ __launch_bounds__(256) void flce_sum_slots(const float4* __restrict__ part,
+                                                      int64_t slots, int64_t nquads,
+                                                      uint2* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (i >= nquads) return;
+  float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int64_t p0 = 0; p0 < slots; p0 += kSumUnroll) {
+    float4 v[kSumUnroll];
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u)
+      v[u] = p0 + u < slots ? part[(p0 + u) * nquads + i] : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int u = 0; u < kSumUnroll; ++u) {
+      s.x += v[u].x;
+      s.y += v[u].y;
+      s.z += v[u].z;
+      s.w += v[u].w;
+    }
+  }
+  bf16x2_t lo = {(__bf16)s.x, (__bf16)s.y};
+  bf16x2_t hi = {(__bf16)s.z, (__bf16)s.w};
+  out[i] = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+}
+
 __global__ __launch_bounds__(256) void fill_zero_u32(uint32_t* __restrict__ p, int64_t n,
                                                      float* __restrict__ loss) {
   const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -758,7 +812,7 @@ inline int64_t logits_ld(int64_t V) { return round_up(V, 8); }
 
 struct Layout {
   int64_t chunk, nchunks, nparts;
-  size_t off_logits, off_stats, off_lse, off_rows, off_misc, off_acc, total;
+  size_t off_logits, off_stats, off_lse, off_rows, off_misc, off_acc, off_part, total;
 };
 
 Layout layout(int64_t N, int64_t H, int64_t V, int64_t chunk, bool grads, bool acc_bf16) {
@@ -779,6 +833,11 @@ Layout layout(int64_t N, int64_t H, int64_t V, int64_t chunk, bool grads, bool a
   l.off_rows = take((size_t)N * 4);
   l.off_misc = take(64);
   l.off_acc = grads && !acc_bf16 && l.nchunks > 1 ? take((size_t)V * H * 4) : 0;
+  // grad_hidden's K slots; the last chunk, with fewer rows, may be cut finer
+  const int64_t last = N - (l.nchunks - 1) * l.chunk;
+  const int64_t pf = ts_plan::hidden_split_bytes(l.nchunks > 1 ? l.chunk : last, H, V);
+  const int64_t pl = ts_plan::hidden_split_bytes(last, H, V);
+  l.off_part = grads ? take((size_t)(pf > pl ? pf : pl)) : 0;
   l.total = off;
   return l;
 }
@@ -788,10 +847,14 @@ Layout layout(int64_t N, int64_t H, int64_t V, int64_t chunk, bool grads, bool a
 // grad_weight 6.93 vs 7.19 ms, bit-identical results. The matrix cores are busier
 // per clock (69-76% against 58-67%); the box's clock under this load drops to
 // 1.55-1.6 GHz from 1.75-1.85, which takes back part of the gain.
+int64_t gemm_pieces(const GemmArgs& a) {
+  return ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN) * (a.splits > 1 ? a.splits : 1);
+}
+
 template <int kMode, int kMA = ts_gemm::kKMajor, int kMB = ts_gemm::kKMajor>
 ts_status launch_gemm(const GemmArgs& a, hipStream_t st, const char* name) {
   constexpr int kW = 8;
-  const int64_t tiles = ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN);
+  const int64_t tiles = gemm_pieces(a);
   if (tiles <= 0) return TS_OK;
   if (tiles > 0x7fffffffLL) return ts_host::fail(TS_ERR_SHAPE, "%s: too many tiles", name);
   hipLaunchKernelGGL((flce_gemm<kMode, kMA, kMB, kW>), dim3((unsigned)tiles),
@@ -803,14 +866,84 @@ template <int kMode1, int kMA1, int kMB1, int kMode2, int kMA2, int kMB2>
 ts_status launch_gemm_pair(const GemmArgs& a1, const GemmArgs& a2, hipStream_t st,
                            const char* name) {
   constexpr int kW = 8;
-  const int64_t t1 = ((a1.M + BM - 1) / BM) * ((a1.N + BN - 1) / BN);
-  const int64_t t2 = ((a2.M + BM - 1) / BM) * ((a2.N + BN - 1) / BN);
+  const int64_t t1 = gemm_pieces(a1);
+  const int64_t t2 = gemm_pieces(a2);
   if (t1 + t2 <= 0) return TS_OK;
   if (t1 + t2 > 0x7fffffffLL) return ts_host::fail(TS_ERR_SHAPE, "%s: too many tiles", name);
   hipLaunchKernelGGL((flce_gemm_pair<kMode1, kMA1, kMB1, kMode2, kMA2, kMB2, kW>),
                      dim3((unsigned)(t1 + t2)), dim3(ts_gemm::Cfg<kW>::kThreads), 0, st, a1, a2,
                      t1);
   return ts_host::check_launch(name);
+}
+
+// The gradient GEMMs of one chunk of dlogits D, grad_hidden (dh, D K-major, the weight
+// MN-major) and grad_weight (dw, both operands MN-major), with the epilogues hmode and
+// wmode: in one grid when both are wanted (C of an unwanted one is NULL), grad_hidden's
+// few long pieces first.
+ts_status launch_grads(const GemmArgs& dh, int hmode, const GemmArgs& dw, int wmode,
+                       hipStream_t st, const char* name) {
+  using ts_gemm::kKMajor;
+  using ts_gemm::kMNMajor;
+  const bool h = dh.C != nullptr, w = dw.C != nullptr;
+#define TS_PAIR(HM, WM)                                                                       \
+  if (h && w && hmode == HM && wmode == WM)                                                   \
+    return launch_gemm_pair<HM, kKMajor, kMNMajor, WM, kMNMajor, kMNMajor>(dh, dw, st, name);
+  TS_PAIR(kEpiBf16, kEpiBf16)
+  TS_PAIR(kEpiBf16, kEpiAddBf16)
+  TS_PAIR(kEpiBf16, kEpiF32)
+  TS_PAIR(kEpiBf16, kEpiAccF32)
+  TS_PAIR(kEpiBf16, kEpiAccBf16)
+  TS_PAIR(kEpiF32, kEpiBf16)
+  TS_PAIR(kEpiF32, kEpiAddBf16)
+  TS_PAIR(kEpiF32, kEpiF32)
+  TS_PAIR(kEpiF32, kEpiAccF32)
+  TS_PAIR(kEpiF32, kEpiAccBf16)
+  TS_PAIR(kEpiAccF32, kEpiBf16)
+  TS_PAIR(kEpiAccBf16, kEpiBf16)
+#undef TS_PAIR
+#define TS_ONE(COND, A, MODE, MA)                                                             \
+  if (COND) return launch_gemm<MODE, MA, kMNMajor>(A, st, name);
+  TS_ONE(h && !w && hmode == kEpiBf16, dh, kEpiBf16, kKMajor)
+  TS_ONE(h && !w && hmode == kEpiF32, dh, kEpiF32, kKMajor)
+  TS_ONE(h && !w && hmode == kEpiAccF32, dh, kEpiAccF32, kKMajor)
+  TS_ONE(h && !w && hmode == kEpiAccBf16, dh, kEpiAccBf16, kKMajor)
+  TS_ONE(!h && w && wmode == kEpiBf16, dw, kEpiBf16, kMNMajor)
+  TS_ONE(!h && w && wmode == kEpiAddBf16, dw, kEpiAddBf16, kMNMajor)
+  TS_ONE(!h && w && wmode == kEpiF32, dw, kEpiF32, kMNMajor)
+  TS_ONE(!h && w && wmode == kEpiAccF32, dw, kEpiAccF32, kMNMajor)
+  TS_ONE(!h && w && wmode == kEpiAccBf16, dw, kEpiAccBf16, kMNMajor)
+#undef TS_ONE
+  if (!h && !w) return TS_OK;
+  return ts_host::fail(TS_ERR_INVALID_ARGUMENT, "%s: no kernel for epilogues %d, %d", name, hmode,
+                       wmode);
+}
+
+// grad_hidden = bf16 of the sum of the K slots' partials [slots][M][H].
+ts_status launch_sum_slots(const float* part, int64_t slots, int64_t M, int64_t H, __bf16* out,
+                           hipStream_t st) {
+  const int64_t nquads = M * H / 4;
+  hipLaunchKernelGGL(flce_sum_slots, dim3((unsigned)((nquads + 255) / 256)), dim3(256), 0, st,
+                     reinterpret_cast<const float4*>(part), slots, nquads,
+                     reinterpret_cast<uint2*>(out));
+  return ts_host::check_launch("flce_sum_slots");
+}
+
+// Both gradients from dlogits that span the whole vocabulary (K of dh): grad_hidden
+// through K slots and their sum when ts_plan::hidden_split cuts K, `part` then being
+// its fp32 partials.
+ts_status launch_grads_full_k(GemmArgs dh, const GemmArgs& dw, int wmode, float* part,
+                              hipStream_t st, const char* name) {
+  const ts_plan::KSplit k = ts_plan::hidden_split(dh.M, dh.N, dh.K);
+  const bool split = dh.C != nullptr && k.splits > 1;
+  if (split) {
+    dh.splits = k.splits;
+    dh.kper = k.kper;
+    dh.C32 = part;
+    dh.ldc32 = dh.N;
+  }
+  const ts_status s = launch_grads(dh, split ? kEpiF32 : kEpiBf16, dw, wmode, st, name);
+  if (s != TS_OK || !split) return s;
+  return launch_sum_slots(part, k.splits, dh.M, dh.N, dh.C, st);
 }
 
 }  // namespace
@@ -887,6 +1020,7 @@ extern "C" ts_status ts_flce_fwd_bwd(const void* hidden, int64_t ldh, const void
   int* n_valid = reinterpret_cast<int*>(ws + lay.off_misc);
   float* scale = reinterpret_cast<float*>(ws + lay.off_misc + 16);
   float* acc32 = reinterpret_cast<float*>(ws + lay.off_acc);
+  float* part = reinterpret_cast<float*>(ws + lay.off_part);
   const __bf16* Hd = static_cast<const __bf16*>(hidden);
   const __bf16* Wd = static_cast<const __bf16*>(weight);
   const int64_t ldl = logits_ld(V);
@@ -925,8 +1059,6 @@ extern "C" ts_status ts_flce_fwd_bwd(const void* hidden, int64_t ldh, const void
     hipLaunchKernelGGL(flce_dlogits, dim3((unsigned)(Mc * dchunks)), dim3(256), 0, st, Lc, ldl,
                        lse_ws + r0, labels + r0, V, dchunks, ignore_index, scale, (int64_t)0);
     TS_TRY(ts_host::check_launch("flce_dlogits"));
-    using ts_gemm::kKMajor;
-    using ts_gemm::kMNMajor;
     GemmArgs dh{};
     dh.A = Lc;  // dlogits [Mc, V], K-major (zero from V to the end of the row's last vector)
     dh.lda = ldl;
@@ -935,7 +1067,7 @@ extern "C" ts_status ts_flce_fwd_bwd(const void* hidden, int64_t ldh, const void
     dh.M = Mc;
     dh.N = H;
     dh.K = V;
-    dh.C = static_cast<__bf16*>(grad_hidden) + r0 * H;
+    dh.C = grad_hidden != nullptr ? static_cast<__bf16*>(grad_hidden) + r0 * H : nullptr;
     dh.ldc = H;
     GemmArgs dw{};
     dw.A = Lc;             // dlogits [Mc, V] as the [V, Mc] operand: MN-major, k = token
@@ -956,32 +1088,7 @@ extern "C" ts_status ts_flce_fwd_bwd(const void* hidden, int64_t ldh, const void
                       : c == 0         ? kEpiF32
                       : c + 1 < lay.nchunks ? kEpiAccF32
                                             : kEpiAccBf16;
-    if (grad_hidden != nullptr && grad_weight != nullptr) {
-      // both gradient GEMMs in one grid (grad_hidden's few long tiles first)
-#define TS_PAIR(WM)                                                                         \
-  TS_TRY((launch_gemm_pair<kEpiBf16, kKMajor, kMNMajor, WM, kMNMajor, kMNMajor>(dh, dw, st,   \
-                                                                                "flce_gemm_grads")))
-      if (wmode == kEpiBf16) TS_PAIR(kEpiBf16);
-      else if (wmode == kEpiAddBf16) TS_PAIR(kEpiAddBf16);
-      else if (wmode == kEpiF32) TS_PAIR(kEpiF32);
-      else if (wmode == kEpiAccF32) TS_PAIR(kEpiAccF32);
-      else TS_PAIR(kEpiAccBf16);
-#undef TS_PAIR
-    } else if (grad_hidden != nullptr) {
-      TS_TRY((launch_gemm<kEpiBf16, kKMajor, kMNMajor>(dh, st, "flce_gemm_dhidden")));
-    } else if (grad_weight != nullptr) {
-      if (wmode == kEpiBf16) {
-        TS_TRY((launch_gemm<kEpiBf16, kMNMajor, kMNMajor>(dw, st, "flce_gemm_dweight")));
-      } else if (wmode == kEpiAddBf16) {
-        TS_TRY((launch_gemm<kEpiAddBf16, kMNMajor, kMNMajor>(dw, st, "flce_gemm_dweight")));
-      } else if (wmode == kEpiF32) {
-        TS_TRY((launch_gemm<kEpiF32, kMNMajor, kMNMajor>(dw, st, "flce_gemm_dweight")));
-      } else if (wmode == kEpiAccF32) {
-        TS_TRY((launch_gemm<kEpiAccF32, kMNMajor, kMNMajor>(dw, st, "flce_gemm_dweight")));
-      } else {
-        TS_TRY((launch_gemm<kEpiAccBf16, kMNMajor, kMNMajor>(dw, st, "flce_gemm_dweight")));
-      }
-    }
+    TS_TRY(launch_grads_full_k(dh, dw, wmode, part, st, "flce_gemm_grads"));
   }
   hipLaunchKernelGGL(flce_loss, dim3(1), dim3(256), 0, st, rows_ws, N, n_valid,
                      reduction == 0 ? 1 : 0, loss, scale);
@@ -1030,6 +1137,7 @@ int64_t bwd_chunk_cols(int64_t V, int64_t chunk_cols) {
 
 struct BwdLayout {
   int64_t chunk, nchunks;
+  int64_t splits;  // K slots of grad_hidden in every chunk (ts_plan::hidden_split of a full one)
   size_t off_d, off_acc, off_dscale, off_misc, total;
 };
 
@@ -1037,6 +1145,7 @@ BwdLayout bwd_layout(int64_t N, int64_t H, int64_t V, int64_t chunk_cols) {
   BwdLayout l{};
   l.chunk = bwd_chunk_cols(V, chunk_cols);
   l.nchunks = (V + l.chunk - 1) / l.chunk;
+  l.splits = ts_plan::hidden_split(N, H, l.chunk < V ? l.chunk : V).splits;
   size_t off = 0;
   auto take = [&](size_t bytes) {
     const size_t o = off;
@@ -1044,7 +1153,8 @@ BwdLayout bwd_layout(int64_t N, int64_t H, int64_t V, int64_t chunk_cols) {
     return o;
   };
   l.off_d = take((size_t)N * (size_t)l.chunk * 2);
-  l.off_acc = l.nchunks > 1 ? take((size_t)N * (size_t)H * 4) : 0;
+  l.off_acc = l.nchunks > 1 || l.splits > 1
+                  ? take((size_t)l.splits * (size_t)N * (size_t)H * 4) : 0;
   l.off_dscale = take((size_t)N * 4);
   l.off_misc = take(64);
   l.total = off;
@@ -1231,8 +1341,6 @@ extern "C" ts_status ts_flce_backward(const void* hidden, int64_t ldh, const voi
   hipLaunchKernelGGL(flce_dscale, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, labels, N,
                      ignore_index, dloss, dloss_stride, n_valid, reduction == 0 ? 1 : 0, dscale);
   TS_TRY(ts_host::check_launch("flce_dscale"));
-  using ts_gemm::kKMajor;
-  using ts_gemm::kMNMajor;
   for (int64_t c = 0; c < lay.nchunks; ++c) {
     const int64_t v0 = c * lay.chunk;
     const int64_t Vc = V - v0 < lay.chunk ? V - v0 : lay.chunk;
@@ -1253,48 +1361,44 @@ extern "C" ts_status ts_flce_backward(const void* hidden, int64_t ldh, const voi
     g.dscale = dscale;
     g.xf = xf;
     TS_TRY(launch_gemm<kEpiDlogits>(g, st, "flce_gemm_dlogits"));
-    if (grad_hidden != nullptr) {
-      // grad_hidden (+)= D [N, Vc] @ W[v0 : v0 + Vc] (the chunk read as the MN-major [H, Vc]
-      // operand); carried in fp32 across chunks and rounded once
-      GemmArgs d{};
-      d.A = D;
-      d.lda = lay.chunk;
-      d.B = Wd + v0 * ldw;
-      d.ldb = ldw;
-      d.M = N;
-      d.N = H;
-      d.K = Vc;
-      d.C = static_cast<__bf16*>(grad_hidden);
-      d.ldc = H;
-      d.C32 = acc32;
-      d.ldc32 = H;
-      if (lay.nchunks == 1) {
-        TS_TRY((launch_gemm<kEpiBf16, kKMajor, kMNMajor>(d, st, "flce_gemm_dhidden")));
-      } else if (c == 0) {
-        TS_TRY((launch_gemm<kEpiF32, kKMajor, kMNMajor>(d, st, "flce_gemm_dhidden")));
-      } else if (c + 1 < lay.nchunks) {
-        TS_TRY((launch_gemm<kEpiAccF32, kKMajor, kMNMajor>(d, st, "flce_gemm_dhidden")));
-      } else {
-        TS_TRY((launch_gemm<kEpiAccBf16, kKMajor, kMNMajor>(d, st, "flce_gemm_dhidden")));
-      }
-    }
-    if (grad_weight != nullptr) {
-      // grad_weight[v0 : v0 + Vc] = D^T @ hidden: D as the MN-major [Vc, N] operand, hidden
-      // as the MN-major [H, N] operand
-      GemmArgs d{};
-      d.A = D;
-      d.lda = lay.chunk;
-      d.B = Hd;
-      d.ldb = ldh;
-      d.M = Vc;
-      d.N = H;
-      d.K = N;
-      d.C = static_cast<__bf16*>(grad_weight) + v0 * H;
-      d.ldc = H;
-      TS_TRY((launch_gemm<kEpiBf16, kMNMajor, kMNMajor>(d, st, "flce_gemm_dweight")));
-    }
+    // grad_hidden (+)= D [N, Vc] @ W[v0 : v0 + Vc] (the chunk read as the MN-major [H, Vc]
+    // operand); carried in fp32 across the chunks, in one slot per K split, and rounded once
+    GemmArgs dh{};
+    dh.A = D;
+    dh.lda = lay.chunk;
+    dh.B = Wd + v0 * ldw;
+    dh.ldb = ldw;
+    dh.M = N;
+    dh.N = H;
+    dh.K = Vc;
+    dh.C = static_cast<__bf16*>(grad_hidden);
+    dh.ldc = H;
+    dh.C32 = acc32;
+    dh.ldc32 = H;
+    dh.splits = lay.splits;
+    dh.kper = ts_plan::split_kper(Vc, lay.splits);
+    const bool last = c + 1 == lay.nchunks;
+    const int hmode = lay.splits > 1 ? (c == 0 ? kEpiF32 : kEpiAccF32)
+                      : lay.nchunks == 1 ? kEpiBf16
+                      : c == 0           ? kEpiF32
+                      : !last            ? kEpiAccF32
+                                         : kEpiAccBf16;
+    // grad_weight[v0 : v0 + Vc] = D^T @ hidden: D as the MN-major [Vc, N] operand, hidden
+    // as the MN-major [H, N] operand
+    GemmArgs dw{};
+    dw.A = D;
+    dw.lda = lay.chunk;
+    dw.B = Hd;
+    dw.ldb = ldh;
+    dw.M = Vc;
+    dw.N = H;
+    dw.K = N;
+    dw.C = grad_weight != nullptr ? static_cast<__bf16*>(grad_weight) + v0 * H : nullptr;
+    dw.ldc = H;
+    TS_TRY(launch_grads(dh, hmode, dw, kEpiBf16, st, "flce_gemm_grads"));
   }
-  return TS_OK;
+  if (grad_hidden == nullptr || lay.splits == 1) return TS_OK;
+  return launch_sum_slots(acc32, lay.splits, N, H, static_cast<__bf16*>(grad_hidden), st);
 }
 
 // The backward from logits the forward kept (ts_flce_forward_keep): dz in place
@@ -1303,7 +1407,7 @@ extern "C" ts_status ts_flce_backward(const void* hidden, int64_t ldh, const voi
 namespace {
 
 struct KeptLayout {
-  size_t off_dscale, off_misc, total;
+  size_t off_dscale, off_misc, off_part, total;
 };
 
 KeptLayout kept_layout(int64_t N) {
@@ -1316,6 +1420,7 @@ KeptLayout kept_layout(int64_t N) {
   };
   l.off_dscale = take((size_t)N * 4);
   l.off_misc = take(64);
+  l.off_part = take((size_t)ts_plan::hidden_split_bytes_any_shape(N));
   l.total = off;
   return l;
 }
@@ -1381,8 +1486,6 @@ extern "C" ts_status ts_flce_backward_kept(const void* hidden, int64_t ldh, cons
   hipLaunchKernelGGL(flce_dlogits_kept, dim3((unsigned)(N * dchunks)), dim3(256), 0, st, L, ldl,
                      lse, labels, V, dchunks, dscale, xf);
   TS_TRY(ts_host::check_launch("flce_dlogits_kept"));
-  using ts_gemm::kKMajor;
-  using ts_gemm::kMNMajor;
   GemmArgs dh{};
   dh.A = L;  // dz [N, V], K-major (rows of ldl, zero from V on)
   dh.lda = ldl;
@@ -1403,12 +1506,8 @@ extern "C" ts_status ts_flce_backward_kept(const void* hidden, int64_t ldh, cons
   dw.K = N;
   dw.C = static_cast<__bf16*>(grad_weight);
   dw.ldc = H;
-  if (grad_hidden != nullptr && grad_weight != nullptr)
-    return launch_gemm_pair<kEpiBf16, kKMajor, kMNMajor, kEpiBf16, kMNMajor, kMNMajor>(
-        dh, dw, st, "flce_gemm_grads_kept");
-  if (grad_hidden != nullptr)
-    return launch_gemm<kEpiBf16, kKMajor, kMNMajor>(dh, st, "flce_gemm_dhidden_kept");
-  return launch_gemm<kEpiBf16, kMNMajor, kMNMajor>(dw, st, "flce_gemm_dweight_kept");
+  return launch_grads_full_k(dh, dw, kEpiBf16, reinterpret_cast<float*>(ws + lay.off_part), st,
+                             "flce_gemm_grads_kept");
 }
 
 // ---------------------------------------------------------------------------
@@ -1420,7 +1519,7 @@ namespace {
 
 struct VocabLayout {
   int64_t nparts;
-  size_t off_logits, off_stats, off_lse, off_rows, off_misc, total;
+  size_t off_logits, off_stats, off_lse, off_rows, off_misc, off_part, total;
 };
 
 VocabLayout vocab_layout(int64_t N, int64_t Vp) {
@@ -1437,6 +1536,7 @@ VocabLayout vocab_layout(int64_t N, int64_t Vp) {
   l.off_lse = take((size_t)N * 4);
   l.off_rows = take((size_t)N * 4);
   l.off_misc = take(64);
+  l.off_part = take((size_t)ts_plan::hidden_split_bytes_any_h(N, Vp));
   l.total = off;
   return l;
 }
@@ -1557,8 +1657,6 @@ extern "C" ts_status ts_flce_vocab_bwd(const void* hidden, int64_t ldh, const vo
   TS_TRY(ts_host::check_launch("flce_dlogits"));
   const __bf16* Hd = static_cast<const __bf16*>(hidden);
   const __bf16* Wd = static_cast<const __bf16*>(weight);
-  using ts_gemm::kKMajor;
-  using ts_gemm::kMNMajor;
   GemmArgs dh{};
   dh.A = L;  // dlogits [N, Vp], K-major (zero from Vp to the end of the row's last vector)
   dh.lda = ldl;
@@ -1579,14 +1677,8 @@ extern "C" ts_status ts_flce_vocab_bwd(const void* hidden, int64_t ldh, const vo
   dw.K = N;
   dw.C = static_cast<__bf16*>(grad_weight_shard);
   dw.ldc = H;
-  if (grad_hidden_partial != nullptr && grad_weight_shard != nullptr) {
-    // both GEMMs read the same dlogits: one grid
-    return launch_gemm_pair<kEpiBf16, kKMajor, kMNMajor, kEpiBf16, kMNMajor, kMNMajor>(
-        dh, dw, st, "flce_vocab_gemm_grads");
-  }
-  if (grad_hidden_partial != nullptr)
-    return launch_gemm<kEpiBf16, kKMajor, kMNMajor>(dh, st, "flce_vocab_gemm_dhidden");
-  return launch_gemm<kEpiBf16, kMNMajor, kMNMajor>(dw, st, "flce_vocab_gemm_dweight");
+  return launch_grads_full_k(dh, dw, kEpiBf16, reinterpret_cast<float*>(ws + lay.off_part), st,
+                             "flce_vocab_gemm_grads");
 }
 
 namespace {

@@ -261,17 +261,74 @@ inline bool magic64_exact(uint64_t n_max, uint64_t d) {
 constexpr int64_t kGemmGroupM = 4;
 constexpr int64_t kXcds = 8;
 
-TS_HOST_DEVICE inline void gemm_tile_of(int64_t bid, int64_t MT, int64_t NT, int64_t& mt,
-                                        int64_t& nt) {
-  const int64_t T = MT * NT;
+// One piece of a GEMM whose K is cut into `splits` slots: slots follow one another
+// in the logical order, so the workgroups an XCD holds work on the same K range and
+// share its operand panels.
+TS_HOST_DEVICE inline void gemm_piece_of(int64_t bid, int64_t MT, int64_t NT, int64_t splits,
+                                         int64_t& slot, int64_t& mt, int64_t& nt) {
+  const int64_t T = MT * NT * splits;
   const int64_t x = bid % kXcds, i = bid / kXcds, q = T / kXcds, r = T % kXcds;
-  const int64_t t = x * q + (x < r ? x : r) + i;  // logical tile
+  const int64_t p = x * q + (x < r ? x : r) + i;  // logical piece
+  slot = p / (MT * NT);
+  const int64_t t = p - slot * (MT * NT);         // logical tile of the slot
   const int64_t per_group = kGemmGroupM * NT;
   const int64_t g = t / per_group;
   const int64_t w = t - g * per_group;
   const int64_t gm = MT - g * kGemmGroupM < kGemmGroupM ? MT - g * kGemmGroupM : kGemmGroupM;
   mt = g * kGemmGroupM + w % gm;
   nt = w / gm;
+}
+TS_HOST_DEVICE inline void gemm_tile_of(int64_t bid, int64_t MT, int64_t NT, int64_t& mt,
+                                        int64_t& nt) {
+  int64_t slot;
+  gemm_piece_of(bid, MT, NT, 1, slot, mt, nt);
+}
+
+// K split of the linear-CE's grad_hidden GEMM, [M, K] @ [K, H] with K the vocabulary (or
+// one chunk of it). Its M x H tiles are few while K is long: at M = 1024, H = 768,
+// K = 50257 it has 12 tiles of 1571 k-blocks each, and 12 CUs work while the others have
+// long finished grad_weight's short tiles. So K is cut into `splits` slots, as many as
+// keep the pieces within one per CU (the grad_weight tiles of the same grid fill what is
+// left), each at least kSplitMinBlocks k-blocks long: a piece writes its fp32 partial
+// tile (256 KB, the time of about 10 k-blocks at a CU's share of HBM), and a second
+// kernel sums the slots in order and rounds once. With a tile for every CU or more there
+// is one slot and nothing changes. The rule looks at M, H and K only, so every schedule
+// sums a given shape in the same order. Measured on MI355X, the gradient GEMMs of the shape
+// above: 1036 us whole, 174 us plus 11.5 us for the sum in 21 slots; of M = 2000, H = 4096,
+// K = 16128 (128 tiles): 566 us in two launches, 447 us in one grid with 2 slots.
+constexpr int64_t kGemmTile = 256;        // M and N of a tile
+constexpr int64_t kGemmBlockK = 32;       // a k-block
+constexpr int64_t kCus = 256;
+constexpr int64_t kSplitMinBlocks = 64;
+struct KSplit {
+  int64_t splits;  // slots, at least 1
+  int64_t kper;    // k per slot, whole k-blocks (the last slot may have fewer, or none)
+};
+// The cut of K into `splits` slots of whole k-blocks.
+TS_HOST_DEVICE inline int64_t split_kper(int64_t K, int64_t splits) {
+  const int64_t blocks = (K + kGemmBlockK - 1) / kGemmBlockK;
+  return (blocks + splits - 1) / splits * kGemmBlockK;
+}
+inline KSplit hidden_split(int64_t M, int64_t H, int64_t K) {
+  const int64_t tiles =
+      ((M + kGemmTile - 1) / kGemmTile) * ((H + kGemmTile - 1) / kGemmTile);
+  const int64_t blocks = (K + kGemmBlockK - 1) / kGemmBlockK;
+  int64_t s = tiles > 0 ? kCus / tiles : 1;
+  if (s > blocks / kSplitMinBlocks) s = blocks / kSplitMinBlocks;
+  if (s < 1) s = 1;
+  return KSplit{s, split_kper(K, s)};
+}
+// Bytes of the fp32 partials of one such GEMM ([splits][M][H]), and a bound on them for
+// any H where a workspace query does not know it (at most one tile per CU when split).
+inline int64_t hidden_split_bytes(int64_t M, int64_t H, int64_t K) {
+  const KSplit k = hidden_split(M, H, K);
+  return k.splits > 1 ? k.splits * M * H * 4 : 0;
+}
+inline int64_t hidden_split_bytes_any_h(int64_t M, int64_t K) {
+  return hidden_split(M, 1, K).splits > 1 ? kCus * kGemmTile * kGemmTile * 4 : 0;
+}
+inline int64_t hidden_split_bytes_any_shape(int64_t M) {
+  return hidden_split_bytes_any_h(M, (int64_t)1 << 40);
 }
 
 // ---------------------------------------------------------------------------
