@@ -115,6 +115,21 @@ template <typename T>
 __device__ inline u32x4 ld16_stream(const T* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(p));
 }
+// The same at any element address: gfx950 runs 16-byte global accesses at 2-byte
+// alignment, and the element-aligned vector type makes the compiler keep them whole.
+typedef u32x4 u32x4_any __attribute__((aligned(2)));
+template <typename T>
+__device__ inline u32x4 ld16_any_stream(const T* p) {
+  return __builtin_nontemporal_load(reinterpret_cast<const u32x4_any*>(p));
+}
+template <typename T>
+__device__ inline void st16_any_stream(T* p, const u32x4& v) {
+  __builtin_nontemporal_store(v, reinterpret_cast<u32x4_any*>(p));
+}
+template <typename T>
+__device__ inline void st16_any(T* p, const u32x4& v) {
+  *reinterpret_cast<u32x4_any*>(p) = v;
+}
 template <typename T>
 __device__ inline void st16(T* p, const u32x4& v) {
   *reinterpret_cast<u32x4*>(p) = v;

@@ -1,0 +1,531 @@
+// Device code shared by the cross-entropy kernels (cross_entropy.hip and the one-pass
+// kernels of ce_fused_*.hip): logit transforms, gradients, the elements after a row's last
+// whole vector, and the one-pass kernel with its launcher. The one-pass kernel has many
+// instantiations (row shapes, modes, alignment), so each data type compiles in its own file.
+#pragma once
+
+#include <math.h>
+
+#include "common.hpp"
+#include "plan.hpp"
+
+namespace ts_ce {
+
+using namespace ts;
+
+// What a kernel applies besides the softmax: nothing, label smoothing, or any of logit
+// scaling, softcapping and smoothing (each tested at run time, uniformly).
+enum Mode : int { kPlain = 0, kSmooth = 1, kGeneral = 2 };
+
+// Logit scaling then softcapping, in the reference's order
+// (kernels/triton_kernels.py:214-217): z = softcap * tanh(scale * x / softcap).
+struct Xform {
+  float scale;    // 1 when off
+  float softcap;  // 0 = off
+  float inv_cap;  // 1 / softcap
+};
+inline Xform make_xform(float logit_scale, float softcap) {
+  return Xform{logit_scale != 0.f ? logit_scale : 1.f, softcap,
+               softcap != 0.f ? 1.f / softcap : 0.f};
+}
+inline Mode mode_of(float logit_scale, float softcap, float smoothing) {
+  return logit_scale != 0.f || softcap != 0.f ? kGeneral : smoothing != 0.f ? kSmooth : kPlain;
+}
+
+// tanh to about one fp32 ulp in two ranges. Below kTanhSmall: x + x^3 P(x^2), P of degree 5
+// fitted for least relative error over [0, 0.75] (1.7e-9 before rounding, 0.75 ulp in fp32
+// arithmetic). From there on: 1 - 2 / (1 + exp(2|x|)) with v_exp_f32 and v_rcp_f32 (each
+// within 1 ulp), whose error the subtraction of a term below 0.37 keeps under 2 ulps. A
+// vector whose values are all small in every lane of the wave skips the second form, which
+// costs twice the first. The device library's tanhf made the softcapped kernels
+// VALU-bound: at [4096, 32000] bf16, softcap 30, the forward took 99 us and now takes 61,
+// the backward 132 and 95.
+constexpr float kTanhSmall = 0.75f;
+__device__ inline float tanh_small(float x) {
+  const float s = x * x;
+  float p = 0.00173693569f;
+  p = __builtin_fmaf(p, s, -0.00765725551f);
+  p = __builtin_fmaf(p, s, 0.0214520339f);
+  p = __builtin_fmaf(p, s, -0.0538927242f);
+  p = __builtin_fmaf(p, s, 0.133326948f);
+  p = __builtin_fmaf(p, s, -0.333333164f);
+  return __builtin_fmaf(p, s * x, x);
+}
+__device__ inline float tanh_large(float x) {
+  const float e = fast_exp2(fabsf(x) * (2.f * kLog2e));
+  return copysignf(__builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + e), 1.f), x);
+}
+// |x| < kTanhSmall is false for NaN, and tanh_large(NaN) is NaN.
+__device__ inline float tanh1(float x) {
+  return fabsf(x) < kTanhSmall ? tanh_small(x) : tanh_large(x);
+}
+
+// t[i] = tanh of the VE values u[i] a lane holds.
+template <int VE>
+__device__ inline void tanh_vec(const float (&u)[VE], float (&t)[VE]) {
+  float um = fabsf(u[0]);
+#pragma unroll
+  for (int i = 1; i < VE; ++i) um = fmaxf(um, fabsf(u[i]));
+#pragma unroll
+  for (int i = 0; i < VE; ++i) t[i] = tanh_small(u[i]);
+  // fmaxf drops a NaN, whose tanh_small is NaN too
+  if (__builtin_amdgcn_ballot_w64(um >= kTanhSmall) != 0) {
+#pragma unroll
+    for (int i = 0; i < VE; ++i)
+      if (!(fabsf(u[i]) < kTanhSmall)) t[i] = tanh_large(u[i]);
+  }
+}
+
+// The transformed value of one logit.
+template <int kMode>
+__device__ inline float xform1(float x, const Xform& f) {
+  if constexpr (kMode == kGeneral) {
+    x *= f.scale;
+    if (f.softcap != 0.f) x = f.softcap * tanh1(x * f.inv_cap);
+  }
+  return x;
+}
+// The same of a vector, in place.
+template <int kMode, int VE>
+__device__ inline void xform_vec(float (&z)[VE], const Xform& f) {
+  if constexpr (kMode == kGeneral) {
+#pragma unroll
+    for (int i = 0; i < VE; ++i) z[i] *= f.scale;
+    if (f.softcap != 0.f) {
+      float u[VE], t[VE];
+#pragma unroll
+      for (int i = 0; i < VE; ++i) u[i] = z[i] * f.inv_cap;
+      tanh_vec<VE>(u, t);
+#pragma unroll
+      for (int i = 0; i < VE; ++i) z[i] = f.softcap * t[i];
+    }
+  }
+}
+
+// Per-row factors of the gradient: dl * (p - [label] (1 - a) - a / V) * dz/dx.
+struct GradRow {
+  float dl;    // upstream gradient of this row
+  float lse2;  // lse * log2(e)
+  float keep;  // 1 - a, what the label's element subtracts
+  float av;    // a / V
+};
+
+// Gradient of one logit x.
+template <int kMode>
+__device__ inline float grad1(float x, bool is_label, const GradRow& r, const Xform& f) {
+  float z = x, dz = 1.f;
+  if constexpr (kMode == kGeneral) {
+    z *= f.scale;
+    dz = f.scale;
+    if (f.softcap != 0.f) {
+      const float t = tanh1(z * f.inv_cap);
+      z = f.softcap * t;
+      dz = (1.f - t * t) * f.scale;
+    }
+  }
+  float g = fast_exp2(__builtin_fmaf(z, kLog2e, -r.lse2));
+  if (is_label) g -= r.keep;
+  if constexpr (kMode != kPlain) g -= r.av;
+  if constexpr (kMode == kGeneral) g *= dz;
+  return r.dl * g;
+}
+
+// Gradients of a vector of logits; `lab` is the label's position in it, if in [0, VE).
+template <int kMode, int VE>
+__device__ inline void grad_vec(const float (&x)[VE], float (&g)[VE], int64_t lab,
+                                const GradRow& r, const Xform& f) {
+  float z[VE], dz[VE];
+#pragma unroll
+  for (int i = 0; i < VE; ++i) z[i] = x[i];
+  if constexpr (kMode == kGeneral) {
+#pragma unroll
+    for (int i = 0; i < VE; ++i) {
+      z[i] *= f.scale;
+      dz[i] = f.scale;
+    }
+    if (f.softcap != 0.f) {
+      float u[VE], t[VE];
+#pragma unroll
+      for (int i = 0; i < VE; ++i) u[i] = z[i] * f.inv_cap;
+      tanh_vec<VE>(u, t);
+#pragma unroll
+      for (int i = 0; i < VE; ++i) {
+        z[i] = f.softcap * t[i];
+        dz[i] = (1.f - t[i] * t[i]) * f.scale;
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < VE; ++i) {
+    float p = fast_exp2(__builtin_fmaf(z[i], kLog2e, -r.lse2));
+    p = i == lab ? p - r.keep : p;
+    if constexpr (kMode != kPlain) p -= r.av;
+    if constexpr (kMode == kGeneral) p *= dz[i];
+    g[i] = r.dl * p;
+  }
+}
+
+// This lane's element after the row's last whole vector, or -1 (ts_plan::tail_col).
+template <int VE>
+__device__ inline int64_t tail_col(int64_t V) {
+  return ts_plan::tail_col(V, (int)threadIdx.x, VE);
+}
+
+// Adds the value z to an online (max, sum of exp) pair; nothing for -inf.
+__device__ inline void fold1(float z, float& m, float& s) {
+  const float mn = __builtin_fmaxf(m, z);
+  if (z != z) {
+    s = z;  // NaN poisons the row
+  } else if (mn != -INFINITY) {
+    s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) + fast_exp2((z - mn) * kLog2e);
+    m = mn;
+  }
+}
+
+// Loss of a row from its lse and (with smoothing) its sum of z; thread 0 only.
+template <int kMode, typename T>
+__device__ inline float row_loss(const T* xr, int64_t label, int64_t V, int64_t ignore_index,
+                                 float l, float sz, float smoothing, const Xform& xf) {
+  const int64_t col = ts_plan::label_col(label, V, ignore_index);  // not ignored here
+  if (col < 0) return __builtin_nanf("");
+  float out = l - xform1<kMode>(Elt<T>::load1(xr + col), xf);
+  if (kMode != kPlain && smoothing != 0.f)
+    out = (1.f - smoothing) * out + smoothing * (l - sz / (float)V);
+  return out;
+}
+
+// ---------------------------------------------------------------------------
+// Forward + backward in one pass ("schedule B"): one row per workgroup, held in
+// registers (kKv 16-byte vectors per thread; ts_plan::ce_fused_plan picks the shape).
+// Each thread folds its vectors into a (max, sum of exp) pair as they arrive; one LDS
+// exchange of the wave pairs gives the lse (a single barrier). The gradient is then
+// written from the same registers: each valid row is read once and every row written
+// once. Ignored rows are written as zeros without being read.
+//
+// Rows on 16-byte boundaries (kAligned) are addressed through buffer resources (base and
+// range in SGPRs, one VGPR of offset per lane), which keeps the 64 data VGPRs of 16 vectors
+// plus the working set inside the 128-VGPR budget of four waves per SIMD; other rows through
+// element-aligned global accesses. Without label
+// smoothing or logit transforms an element's gradient is
+// exp2(z*log2e - (lse*log2e - log2|dl|)) with the sign of dl applied to the
+// packed result, one FMA and one exp per element; the label element is
+// corrected by the one lane that holds it.
+// ---------------------------------------------------------------------------
+
+// Row lse (and, with smoothing, the row sum of z) from every thread's online
+// (max, sum of exp) pair. lds holds 3 * kNW floats. One barrier: the
+// caller must not write lds again without another barrier in between.
+template <int kMode, int kNW>
+__device__ inline float fused_lse(float m, float s, float& sz, float* lds) {
+  const float wm = wave_max(m);
+  const float ws = wave_sum(s == 0.f ? 0.f : s * fast_exp2((m - wm) * kLog2e));
+  const int wid = threadIdx.x / kWave;
+  if constexpr (kMode != kPlain) sz = wave_sum(sz);
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    lds[wid] = wm;
+    lds[kNW + wid] = ws;
+    if constexpr (kMode != kPlain) lds[2 * kNW + wid] = sz;
+  }
+  __syncthreads();
+  float gm = lds[0];
+#pragma unroll
+  for (int i = 1; i < kNW; ++i) gm = fmaxf(gm, lds[i]);
+  float gs = 0.f, gz = 0.f;
+#pragma unroll
+  for (int i = 0; i < kNW; ++i) {
+    const float si = lds[kNW + i];
+    gs += si == 0.f ? 0.f : si * fast_exp2((lds[i] - gm) * kLog2e);
+    if constexpr (kMode != kPlain) gz += lds[2 * kNW + i];
+  }
+  if constexpr (kMode != kPlain) sz = gz;
+  return gm + logf(gs);
+}
+
+template <typename G>
+constexpr uint32_t sign_bits() {
+  return sizeof(G) == 4 ? 0x80000000u : 0x80008000u;
+}
+
+// Waves per SIMD the register budget must allow: four at 16 vectors per thread (128 VGPRs),
+// six at 8 and eight at 4.
+constexpr int fused_waves(int kv) { return kv >= 16 ? 4 : kv >= 8 ? 6 : 8; }
+
+template <typename T, typename G, int kMode, int kThr, int kKv, bool kAligned>
+__global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(fused_waves(kKv))))
+void ce_fused_vec(
+    const T* __restrict__ logits, int64_t ld, const int64_t* __restrict__ labels, int64_t V,
+    int nvec, int64_t ignore_index, Xform xf, float smoothing, const float* __restrict__ dloss,
+    int64_t dloss_stride, float dloss_scale, float* __restrict__ loss, float* __restrict__ lse_out,
+    G* __restrict__ grad, int64_t ld_grad) {
+  constexpr int VE = Elt<T>::kVec;
+  constexpr int kNW = kThr / kWave;
+  constexpr int kGradBytes = VE * (int)sizeof(G);  // grad bytes per logits vector
+  __shared__ float lds[3 * kNW];
+  const int64_t row = blockIdx.x;
+  const int64_t label = labels[row];
+  const T* xr = logits + row * ld;
+  G* gr = grad + row * ld_grad;
+  // Byte offset of this thread's k-th vector, past the last one an offset no row resource
+  // covers (ts_plan::vec_boffset: the hardware drops such stores, loads read 0).
+  auto voff = [&](int k, int vec_bytes) {
+    return ts_plan::vec_boffset(ts_plan::chunk_vec(0, k, threadIdx.x, kThr, kKv), nvec,
+                                vec_bytes);
+  };
+  const Rsrc go = buf_rsrc(gr, (uint32_t)nvec * kGradBytes);
+  // Stores the gradients of this thread's k-th vector (p1 the second half of fp32 ones).
+  auto store = [&](int k, const u32x4& p0, const u32x4& p1) {
+    if constexpr (kAligned) {
+      const int off = voff(k, kGradBytes);
+      buf_st16_stream(p0, go, off);
+      if constexpr (kGradBytes == 32) buf_st16_stream(p1, go, off + 16);
+    } else {
+      const int v = (int)threadIdx.x + k * kThr;
+      // Not streaming stores: the waves' stores meet inside cache lines here, which L2 should
+      // merge (407 us against 416 us for the [8191, 50257] bf16 loss and gradient).
+      if (v < nvec) {
+        st16_any(gr + v * VE, p0);
+        if constexpr (kGradBytes == 32) st16_any(gr + v * VE + 4, p1);
+      }
+    }
+  };
+  const bool has_tail = V % VE != 0;  // uniform: rows of whole vectors skip its code
+  if (label == ignore_index) {
+    const u32x4 zero = {0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < kKv; ++k) store(k, zero, zero);
+    if (has_tail) {
+      const int64_t ec = tail_col<VE>(V);
+      if (ec >= 0) Elt<G>::store1(gr + ec, 0.f);
+    }
+    if (threadIdx.x == 0) {
+      loss[row] = 0.f;
+      lse_out[row] = 0.f;
+    }
+    return;
+  }
+  // The tail element goes out first: a wait for it later leaves the vectors' loads in
+  // flight. Lanes without one read outside the resource, which touches no memory.
+  const int64_t ec = has_tail ? tail_col<VE>(V) : -1;
+  T xe;
+  {
+    const Rsrc xt = buf_rsrc(xr, (uint32_t)V * (uint32_t)sizeof(T));
+    const int off = ec >= 0 ? (int)(ec * (int64_t)sizeof(T)) : kBufOob;
+    if constexpr (sizeof(T) == 4) {
+      const uint32_t q = __builtin_amdgcn_raw_buffer_load_b32(xt, off, 0, kBufNt);
+      xe = __builtin_bit_cast(T, q);
+    } else {
+      const uint16_t q = __builtin_amdgcn_raw_buffer_load_b16(xt, off, 0, kBufNt);
+      xe = __builtin_bit_cast(T, q);
+    }
+  }
+  u32x4 buf[kKv];
+  if constexpr (kAligned) {
+    const Rsrc xi = buf_rsrc(xr, (uint32_t)nvec * 16u);
+#pragma unroll
+    for (int k = 0; k < kKv; ++k) buf[k] = buf_ld16_stream(xi, voff(k, 16));
+  } else if (nvec > 0) {
+    // unconditional, so that the loads have no branches between them: a lane past the
+    // row's last vector loads its first one, which nothing uses
+#pragma unroll
+    for (int k = 0; k < kKv; ++k) {
+      const int v = (int)threadIdx.x + k * kThr;
+      buf[k] = ld16_any_stream(xr + (v < nvec ? v * VE : 0));
+    }
+  }
+  // Each lane sums exp(z - m) over its vectors against one reference m, the
+  // largest value of its first vector (0 if that vector is all -inf): per
+  // element one unpack, one FMA, one exp and one add, with no running max or
+  // rescale. The sum is exact (terms that underflow lie below the resolution
+  // of a sum that holds exp(0) = 1) unless it ends outside [0.5, inf): a
+  // value more than 88 above m overflowed it, a NaN reached it, or an all
+  // -inf first vector left a sum of values far below 0. Such a lane (only
+  // with extreme logits) folds its vectors again from the registers with an
+  // exact online max and rescale. Lanes without vectors keep m = -inf, s = 0.
+  float m = -INFINITY, mb = 0.f, s = 0.f, sz = 0.f;
+  auto sum_exp = [&](const float (&z)[VE], float bias) {
+    float cs = fast_exp2(__builtin_fmaf(z[0], kLog2e, -bias));
+#pragma unroll
+    for (int i = 1; i < VE; ++i) cs += fast_exp2(__builtin_fmaf(z[i], kLog2e, -bias));
+    return cs;
+  };
+  auto values = [&](const u32x4& q, float (&z)[VE]) {
+    Elt<T>::unpack(q, z);
+    xform_vec<kMode, VE>(z, xf);
+  };
+  auto vmax = [&](const float (&z)[VE]) {
+    float cm = z[0];
+#pragma unroll
+    for (int i = 1; i < VE; ++i) cm = __builtin_fmaxf(cm, z[i]);
+    return cm;
+  };
+  auto fold = [&](const u32x4& q, bool first) {
+    float z[VE];
+    values(q, z);
+    if constexpr (kMode != kPlain) {
+#pragma unroll
+      for (int i = 0; i < VE; ++i) sz += z[i];
+    }
+    if (first) {
+      const float cm = vmax(z);
+      m = cm == -INFINITY ? 0.f : cm;
+      mb = m * kLog2e;
+    }
+    s += sum_exp(z, mb);
+  };
+#pragma unroll
+  for (int k = 0; k < kKv; ++k) {
+    // Vectors every thread holds take a uniform branch; only the row's last
+    // partial sweep tests each lane.
+    if ((k + 1) * kThr <= nvec) fold(buf[k], k == 0);
+    else if ((int)threadIdx.x + k * kThr < nvec) fold(buf[k], k == 0);
+  }
+  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s < INFINITY)) {
+    m = -INFINITY;
+    s = 0.f;
+#pragma unroll
+    for (int k = 0; k < kKv; ++k) {
+      if ((int)threadIdx.x + k * kThr < nvec) {
+        float z[VE];
+        values(buf[k], z);
+        const float mn = __builtin_fmaxf(m, vmax(z));
+        if (mn != -INFINITY) {
+          s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) + sum_exp(z, mn * kLog2e);
+          m = mn;
+        }
+      }
+    }
+  }
+  if (has_tail && ec >= 0) {
+    const float ze = xform1<kMode>(Elt<T>::load1(&xe), xf);
+    fold1(ze, m, s);
+    if constexpr (kMode != kPlain) sz += ze;
+  }
+  const float l = fused_lse<kMode, kNW>(m, s, sz, lds);
+  // The gradient pass re-unpacks the stored vectors; this keeps the compiler
+  // from carrying the first pass's unpacked floats (twice the registers).
+#pragma unroll
+  for (int k = 0; k < kKv; ++k) asm volatile("" : "+v"(buf[k]));
+  if (threadIdx.x == 0) {
+    loss[row] = row_loss<kMode>(xr, label, V, ignore_index, l, sz, smoothing, xf);
+    lse_out[row] = l;
+  }
+  // One upstream gradient per row, moved to a scalar register: its sign below
+  // is then a wave-uniform mask (one XOR per packed dword, no per-lane select).
+  GradRow r;
+  r.dl = __builtin_bit_cast(
+      float, __builtin_amdgcn_readfirstlane(
+                 __builtin_bit_cast(int, dloss[row * dloss_stride] * dloss_scale)));
+  r.lse2 = l * kLog2e;
+  r.keep = 1.f - smoothing;
+  r.av = smoothing / (float)V;
+  if (has_tail && ec >= 0) Elt<G>::store1(gr + ec, grad1<kMode>(Elt<T>::load1(&xe), ec == label, r, xf));
+  // The position of the label is uniform over the workgroup: its correction is a
+  // uniform branch, and only the lane holding the label runs it.
+  const bool lab_in = label >= 0 && label < (int64_t)nvec * VE;
+  const int64_t la = lab_in ? label : 0;
+  const int klab = lab_in ? (int)(la / VE / kThr) : -1;
+  const int tlab = lab_in ? (int)(la / VE % kThr) : -1;
+  const int elab = lab_in ? (int)(la % VE) : 0;
+  const float adl = fabsf(r.dl);
+  const float l2d = r.lse2 - __builtin_amdgcn_logf(adl);  // v_log_f32 is log2
+  const uint32_t smask = kMode == kPlain && (__builtin_bit_cast(uint32_t, r.dl) >> 31) != 0
+                             ? sign_bits<G>() : 0u;
+#pragma unroll
+  for (int k = 0; k < kKv; ++k) {
+    float z[VE], g[VE];
+    Elt<T>::unpack(buf[k], z);
+    if constexpr (kMode == kPlain) {
+#pragma unroll
+      for (int i = 0; i < VE; ++i) g[i] = fast_exp2(__builtin_fmaf(z[i], kLog2e, -l2d));
+      if (k == klab && (int)threadIdx.x == tlab) {
+#pragma unroll
+        for (int i = 0; i < VE; ++i)
+          if (i == elab) g[i] = adl * (fast_exp2(__builtin_fmaf(z[i], kLog2e, -r.lse2)) - 1.f);
+      }
+    } else {
+      grad_vec<kMode, VE>(z, g, -1, r, xf);
+      if (k == klab && (int)threadIdx.x == tlab) {
+#pragma unroll
+        for (int i = 0; i < VE; ++i)
+          if (i == elab) g[i] = grad1<kMode>(z[i], true, r, xf);
+      }
+    }
+    if constexpr (kGradBytes == 32) {
+      u32x4 p0 = Elt<float>::pack(g), p1 = Elt<float>::pack(g + 4);
+      p0 ^= smask;
+      p1 ^= smask;
+      store(k, p0, p1);
+    } else {
+      u32x4 p = Elt<G>::pack(g);
+      p ^= smask;
+      store(k, p, p);
+    }
+  }
+}
+
+// The one-pass kernel for logits of one type (T) with gradients of that type, or fp32 ones of
+// 16-bit logits (`wide`); false, and nothing launched, when no workgroup holds the row.
+struct FusedArgs {
+  const void* logits;
+  int64_t ld;
+  const int64_t* labels;
+  int64_t N, V, ignore_index;
+  Xform xf;
+  Mode mode;
+  float smoothing;
+  const float* dloss;
+  int64_t dloss_stride;
+  float dloss_scale;
+  float* loss;
+  float* lse;
+  void* grad;
+  int64_t ld_grad;
+  hipStream_t st;
+};
+bool fused_bf16(const FusedArgs& a, bool wide, ts_status* status);
+bool fused_f16(const FusedArgs& a, bool wide, ts_status* status);
+bool fused_f32(const FusedArgs& a, ts_status* status);
+
+// Schedule B when the row fits the registers of one workgroup; returns false (nothing
+// launched) otherwise.
+template <typename T, typename G>
+bool launch_fused(const FusedArgs& a, ts_status* status) {
+  constexpr int VE = sizeof(T) == 4 ? 4 : 8;
+  const ts_plan::CeFusedPlan plan = ts_plan::ce_fused_plan(a.V / VE, sizeof(G) != sizeof(T));
+  if (plan.threads == 0 || a.N > INT32_MAX) return false;
+  const bool aligned = ts_host::aligned16(a.logits) && ts_host::aligned16(a.grad) &&
+                       a.ld * (int64_t)sizeof(T) % 16 == 0 &&
+                       a.ld_grad * (int64_t)sizeof(G) % 16 == 0;
+#define TS_CE_FUSED(M, THR, KV, AL)                                                            \
+  if (a.mode == M && plan.threads == THR && plan.kv == KV && aligned == AL) {                  \
+    hipLaunchKernelGGL((ce_fused_vec<T, G, M, THR, KV, AL>), dim3((unsigned)a.N), dim3(THR),   \
+                       0, a.st, static_cast<const T*>(a.logits), a.ld, a.labels, a.V,          \
+                       (int)(a.V / VE), a.ignore_index, a.xf, a.smoothing, a.dloss,            \
+                       a.dloss_stride, a.dloss_scale, a.loss, a.lse, static_cast<G*>(a.grad),  \
+                       a.ld_grad);                                                             \
+    *status = ts_host::check_launch("ce_fused_vec");                                           \
+    return true;                                                                               \
+  }
+#define TS_CE_FUSED_MODES(THR, KV)         \
+  TS_CE_FUSED(kPlain, THR, KV, true)       \
+  TS_CE_FUSED(kSmooth, THR, KV, true)      \
+  TS_CE_FUSED(kGeneral, THR, KV, true)     \
+  TS_CE_FUSED(kPlain, THR, KV, false)      \
+  TS_CE_FUSED(kSmooth, THR, KV, false)     \
+  TS_CE_FUSED(kGeneral, THR, KV, false)
+  if constexpr (sizeof(G) == sizeof(T)) {
+    TS_CE_FUSED_MODES(64, 4)
+    TS_CE_FUSED_MODES(256, 4)
+    TS_CE_FUSED_MODES(256, 8)
+    TS_CE_FUSED_MODES(256, 16)
+    TS_CE_FUSED_MODES(512, 16)
+  }
+  TS_CE_FUSED_MODES(1024, 16)
+#undef TS_CE_FUSED_MODES
+#undef TS_CE_FUSED
+  *status = ts_host::fail(TS_ERR_INVALID_ARGUMENT, "ce_fwd_bwd: no kernel for %d x %d",
+                          plan.threads, plan.kv);
+  return true;
+}
+
+}  // namespace ts_ce

@@ -368,6 +368,37 @@ TS_HOST_DEVICE inline int32_t vec_boffset(int64_t v, int64_t nvec, int vec_bytes
   return v >= 0 && v < nvec ? (int32_t)(v * vec_bytes) : kNoAccess;
 }
 
+// Column of the element that lane t of a row's workgroup holds besides its vectors: the
+// V % VE elements after the row's last whole vector of VE go to the first lanes, one each;
+// -1 for the other lanes.
+TS_HOST_DEVICE inline int64_t tail_col(int64_t V, int t, int VE) {
+  const int64_t c = V / VE * VE + t;
+  return t < VE && c < V ? c : -1;
+}
+
+// Workgroup shape of the one-pass cross-entropy for rows of up to nvec vectors: `threads`
+// lanes of `kv` register vectors hold the row, {0, 0} when no shape does. The smallest
+// workgroup of 16 vectors per thread that holds the row: a CU's registers hold four, two
+// or one of them, so a short row leaves room for others, whose loads and stores then
+// overlap this one's arithmetic and barrier. Rows of up to 2048 vectors take fewer vectors
+// per thread, rows of up to 256 a single wave (no barrier between waves to wait for).
+// Measured on MI355X (bf16, loss and gradient) against 1024 threads x 16 for every row:
+// [16384, 1000] 549 -> 17 us, [16384, 8192] 597 -> 87, [12500, 32000] 492 -> 279,
+// [6103, 65536] 312 -> 273; [16384, 128256] is the same kernel as before. fp32 gradients of 16-bit logits (`wide_grad`), which no
+// training path asks for, keep the one shape that holds every row.
+struct CeFusedPlan {
+  int threads, kv;
+};
+inline CeFusedPlan ce_fused_plan(int64_t nvec, bool wide_grad) {
+  if (nvec > 1024 * 16) return CeFusedPlan{0, 0};
+  if (wide_grad || nvec > 512 * 16) return CeFusedPlan{1024, 16};
+  if (nvec > 256 * 16) return CeFusedPlan{512, 16};
+  if (nvec > 256 * 8) return CeFusedPlan{256, 16};
+  if (nvec > 256 * 4) return CeFusedPlan{256, 8};
+  if (nvec > 64 * 4) return CeFusedPlan{256, 4};
+  return CeFusedPlan{64, 4};
+}
+
 // Row owned by wave `wave` of workgroup `block` in a one-wave-per-row kernel
 // with `waves` row waves per workgroup (flce_rows); such a kernel returns,
 // wave-uniformly, for rows at or past its row count.
