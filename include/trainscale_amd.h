@@ -266,6 +266,25 @@ ts_status ts_ce_bwd(const void* logits, int64_t ld, ts_dtype dtype,
                     ts_stream_t stream);
 
 /*
+ * The reductions around ts_ce_fwd_bwd's per-row losses, one launch each, no
+ * host synchronisation. reduction: 0 mean over the rows whose label is not
+ * ignore_index (at least 1), 1 sum, 2 mean over all rows (at least 1).
+ * ts_ce_loss_weight: *weight = d(reduced loss)/d(row loss) * (hint ? *hint : 1),
+ *   the one-element dloss of ts_ce_fwd_bwd; *used (optional) = the hint factor.
+ * ts_ce_reduce_loss: *loss = the reduced loss of loss_rows [N] (summed in
+ *   double, divided in fp32).
+ * labels: int64 [N]; read for reduction 0 only. All results are fp32 device
+ * scalars; N = 0 gives loss 0. Replaces the reduction and the scale of
+ * FusedCrossEntropyFunction (loss/sota_losses.py:437-532).
+ */
+ts_status ts_ce_loss_weight(const int64_t* labels, int64_t N, int64_t ignore_index,
+                            int32_t reduction, const float* hint, float* weight, float* used,
+                            ts_stream_t stream);
+ts_status ts_ce_reduce_loss(const float* loss_rows, const int64_t* labels, int64_t N,
+                            int64_t ignore_index, int32_t reduction, float* loss,
+                            ts_stream_t stream);
+
+/*
  * ts_ce_fwd and ts_ce_bwd in one pass when the upstream gradient is known at
  * forward time (dloss as for ts_ce_bwd): loss[r], lse[r] and grad as those two
  * functions define them. Each valid row is read once and every row of grad

@@ -73,6 +73,8 @@ SIGNATURES = {
     "ts_ce_fwd": ([P, I64, I32, P, I64, I64, I64, F32, F32, F32, P, P, P], I32),
     "ts_ce_bwd": ([P, I64, I32, P, P, P, I64, F32, P, I64, I32, I64, I64, I64, F32, F32, F32, P],
                   I32),
+    "ts_ce_loss_weight": ([P, I64, I64, I32, P, P, P, P], I32),
+    "ts_ce_reduce_loss": ([P, P, I64, I64, I32, P, P], I32),
     "ts_ce_fwd_bwd": ([P, I64, I32, P, I64, I64, I64, F32, F32, F32, P, I64, F32, P, P, P, I64,
                        I32, P], I32),
     "ts_ce_vocab_shard_stats": ([P, I64, I32, P, I64, I64, I64, P, P], I32),

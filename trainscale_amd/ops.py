@@ -344,6 +344,41 @@ def ce_forward_backward(logits2d: Tensor, ld: int, labels: Tensor, dloss: Tensor
     return loss, lse, grad
 
 
+CE_REDUCTIONS = {"mean": 0, "sum": 1, "batchmean": 2}
+
+
+def ce_loss_weight(labels: Tensor, n: int, ignore_index: int, reduction: str,
+                   hint: Optional[Tensor] = None) -> Tuple[Tensor, Optional[Tensor]]:
+    """(weight, used): d(reduced loss)/d(row loss) times `hint` (a one-element fp32 device
+    tensor, else 1), and a copy of the hint (None without one); one-element fp32 tensors,
+    formed on the device. labels: [n]."""
+    dev = _lib.require_gpu("cross_entropy", labels, hint)
+    labels = _labels(labels, n)
+    out = torch.empty((2,), dtype=torch.float32, device=dev)
+    weight, used = out[:1], out[1:] if hint is not None else None
+    lib = _lib.load()
+    with _lib.on_device(dev):
+        check(lib.ts_ce_loss_weight(ptr(labels), n, int(ignore_index), CE_REDUCTIONS[reduction],
+                                    ptr(hint), ptr(weight), ptr(used), _lib.stream_handle(dev)),
+              "ts_ce_loss_weight")
+    return weight, used
+
+
+def ce_reduce_loss(loss_rows: Tensor, labels: Tensor, ignore_index: int,
+                   reduction: str) -> Tensor:
+    """The per-row losses [n] (fp32, contiguous) reduced to a 0-d fp32 tensor on the device."""
+    dev = _lib.require_gpu("cross_entropy", loss_rows, labels)
+    n = loss_rows.shape[0]
+    labels = _labels(labels, n)
+    loss = torch.empty((), dtype=torch.float32, device=dev)
+    lib = _lib.load()
+    with _lib.on_device(dev):
+        check(lib.ts_ce_reduce_loss(ptr(loss_rows), ptr(labels), n, int(ignore_index),
+                                    CE_REDUCTIONS[reduction], ptr(loss),
+                                    _lib.stream_handle(dev)), "ts_ce_reduce_loss")
+    return loss
+
+
 # ---------------------------------------------------------------------------
 # Vocabulary-parallel cross entropy (the kernels of one rank)
 # ---------------------------------------------------------------------------
