@@ -47,15 +47,33 @@ __device__ inline void load_w(const W* __restrict__ w, int64_t e, float* f) {
   }
 }
 
+// Sum of v over groups of TPR <= 64 consecutive lanes; all 64 lanes active.
+template <int TPR>
+__device__ inline float lanes_sum(float v) {
+  static_assert(TPR == 8 || TPR == 16 || TPR == 32 || TPR == kWave, "lanes per row");
+  if constexpr (TPR == kWave) {
+    return wave_sum(v);
+  } else {
+    v += dpp_f<0xB1>(v);                          // quad_perm [1,0,3,2]
+    v += dpp_f<0x4E>(v);                          // quad_perm [2,3,0,1]
+    v += dpp_f<0x141>(v);                         // row_half_mirror: 8 lanes
+    if constexpr (TPR >= 16) v += dpp_f<0x140>(v);  // row_mirror: 16 lanes
+    if constexpr (TPR == 32)                      // ds_swizzle, lane ^ 16
+      v += __builtin_bit_cast(
+          float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, v), 0x401F));
+    return v;
+  }
+}
+
 // Sum of v over the TPR threads that own one row. `red` holds one float per
 // wave of the workgroup; contains one barrier when TPR > 64 (every thread of
 // the workgroup must call it).
 template <int TPR, int kBlock>
 __device__ inline float row_reduce(float v, float* red) {
-  v = wave_sum(v);
-  if constexpr (TPR == kWave) {
-    return v;
+  if constexpr (TPR <= kWave) {
+    return lanes_sum<TPR>(v);
   } else {
+    v = wave_sum(v);
     constexpr int kWavesPerRow = TPR / kWave;
     const int wid = threadIdx.x / kWave;
     if ((threadIdx.x & (kWave - 1)) == 0) red[wid] = v;
@@ -326,6 +344,109 @@ __global__ __launch_bounds__(512) void rms_bwd_reg(
             make_float4(acc[k][4 * h], acc[k][4 * h + 1], acc[k][4 * h + 2], acc[k][4 * h + 3]);
       }
     }
+  }
+}
+
+// ---------------------------------------------------------------------------
+// Backward of rows of up to 64 vectors (ts_plan::rms_bwd_narrow_plan): TPR lanes per row, one
+// vector each, kNarrowBlock / TPR rows per workgroup and step. A row's sum stays inside the
+// wave, so the loop has no barrier and the 32 waves of a CU (two workgroups, 64 VGPRs a
+// lane) keep HBM busy by themselves: 64 KB of x and dy in flight. The walk over the rows is
+// rms_bwd_reg's. At the end the workgroup's row slots are summed in LDS in a fixed order into
+// one dW partial row, which keeps the second kernel's sum over partial rows short.
+// ---------------------------------------------------------------------------
+template <typename T, typename W, int TPR>
+__global__ __launch_bounds__(ts_plan::kNarrowBlock) __attribute__((amdgpu_waves_per_eu(8)))
+void rms_bwd_narrow(const T* __restrict__ dy, int64_t lddy, const T* __restrict__ x, int64_t ldx,
+                    const W* __restrict__ w, const float* __restrict__ rstd_in,
+                    T* __restrict__ dx, int64_t lddx, float* __restrict__ partial, int64_t rows,
+                    int64_t steps, int nvec, float fcols) {
+  constexpr int V = Elt<T>::kVec;
+  constexpr int kBlock = ts_plan::kNarrowBlock;
+  constexpr int kRpb = kBlock / TPR;
+  __shared__ float4 dw_lds[kBlock * V / 4];
+  const int sub = threadIdx.x / TPR;
+  const int t = threadIdx.x % TPR;
+  const bool in_row = t < nvec;
+  float wf[V], acc[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    acc[i] = 0.f;
+    wf[i] = 1.f;
+  }
+  if (w != nullptr && in_row) load_w<W, V>(w, (int64_t)t * V, wf);
+  const int64_t row0 = (int64_t)blockIdx.x * kRpb + sub;
+  const int64_t rstep = (int64_t)gridDim.x * kRpb;
+  for (int64_t st = 0; st < steps; ++st) {
+    const int64_t row = row0 + st * rstep;
+    const bool valid = row < rows;
+    // a lane with nothing to load reads the matrix's first element (as rms_bwd_reg)
+    u32x4 xv = ld16_stream(x + ts_plan::rms_bwd_load_offset(row0, st, rstep, steps, rows, t, 0,
+                                                            TPR, V, nvec, ldx));
+    u32x4 dv = ld16_stream(dy + ts_plan::rms_bwd_load_offset(row0, st, rstep, steps, rows, t, 0,
+                                                             TPR, V, nvec, lddy));
+    const float rs = rstd_in[valid ? row : 0];
+    const bool ok = valid && in_row;
+    const u32x4 zero = {0, 0, 0, 0};
+    xv = ok ? xv : zero;
+    dv = ok ? dv : zero;
+    const float rstd = valid ? rs : 0.f;
+    float xf[V], df[V];
+    Elt<T>::unpack(xv, xf);
+    Elt<T>::unpack(dv, df);
+    float s = 0.f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const float xh = xf[i] * rstd;
+      s = __builtin_fmaf(df[i] * wf[i], xh, s);
+      acc[i] = __builtin_fmaf(df[i], xh, acc[i]);
+    }
+    const float c1 = lanes_sum<TPR>(s) / fcols;  // every lane active: `steps` is uniform
+    if (ok) {
+      float o[V];
+#pragma unroll
+      for (int i = 0; i < V; ++i) o[i] = rstd * (df[i] * wf[i] - (xf[i] * rstd) * c1);
+      st16_stream(dx + row * lddx + (int64_t)t * V, Elt<T>::pack(o));
+    }
+  }
+
+  if (partial == nullptr) return;  // dW not requested
+  // row slots [kRpb][nq quads], summed by groups of nq threads: group g takes the slots
+  // g, g + groups, ..., then the first nq threads the groups' sums
+  const int nq = nvec * V / 4;
+  if (in_row) {
+#pragma unroll
+    for (int h = 0; h < V / 4; ++h)
+      dw_lds[sub * nq + t * (V / 4) + h] =
+          make_float4(acc[4 * h], acc[4 * h + 1], acc[4 * h + 2], acc[4 * h + 3]);
+  }
+  __syncthreads();
+  const int groups = kBlock / nq < kRpb ? kBlock / nq : kRpb;
+  const int g = threadIdx.x / nq;
+  const int q = threadIdx.x - g * nq;
+  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (g < groups) {
+    for (int j = g; j < kRpb; j += groups) {
+      const float4 u = dw_lds[j * nq + q];
+      a.x += u.x;
+      a.y += u.y;
+      a.z += u.z;
+      a.w += u.w;
+    }
+  }
+  __syncthreads();
+  if (g < groups) dw_lds[g * nq + q] = a;
+  __syncthreads();
+  if ((int)threadIdx.x < nq) {
+    float4 b = dw_lds[threadIdx.x];
+    for (int j = 1; j < groups; ++j) {
+      const float4 u = dw_lds[j * nq + threadIdx.x];
+      b.x += u.x;
+      b.y += u.y;
+      b.z += u.z;
+      b.w += u.w;
+    }
+    reinterpret_cast<float4*>(partial + (int64_t)blockIdx.x * nvec * V)[threadIdx.x] = b;
   }
 }
 
@@ -668,7 +789,11 @@ ts_status fwd_typed(const void* x, int64_t ldx, const void* w, void* y, int64_t 
   const W* wp = static_cast<const W*>(w);
   T* yp = static_cast<T*>(y);
   const int64_t nvec = cols / V;
-  const ts_plan::RmsRowPlan plan = ts_plan::rms_fwd_plan(nvec);
+  ts_plan::RmsRowPlan plan = ts_plan::rms_fwd_plan(nvec);
+  if (const int tpr = ts_plan::rms_narrow_tpr(nvec)) {
+    plan.tpr = tpr;
+    plan.rpb = plan.block / tpr;
+  }
   const bool add_ok = !kAdd || (vec_ok<T, W>(add.r, add.ldr, cols, nullptr) &&
                                 (add.h == nullptr || vec_ok<T, W>(add.h, add.ldh, cols, nullptr)));
   if (vec_ok<T, W>(x, ldx, cols, w) && vec_ok<T, W>(y, ldy, cols, nullptr) && add_ok &&
@@ -682,6 +807,9 @@ ts_status fwd_typed(const void* x, int64_t ldx, const void* w, void* y, int64_t 
                        yp, ldy, rstd, rows, (int)nvec, (float)cols, eps, twice, add);          \
     launched = true;                                                                           \
   }
+    TS_LAUNCH_FWD(8, 1)
+    TS_LAUNCH_FWD(16, 1)
+    TS_LAUNCH_FWD(32, 1)
     TS_LAUNCH_FWD(64, 1)
     TS_LAUNCH_FWD(64, 2)
     TS_LAUNCH_FWD(128, 2)
@@ -711,12 +839,35 @@ ts_status bwd_typed(const void* dy, int64_t lddy, const void* x, int64_t ldx, co
   const int64_t nvec = cols / V;
   const bool vec = vec_ok<T, W>(x, ldx, cols, w) && vec_ok<T, W>(dy, lddy, cols, nullptr) &&
                    vec_ok<T, W>(dx, lddx, cols, nullptr);
-  const ts_plan::RmsBwdPlan plan =
+  ts_plan::RmsBwdPlan plan =
       ts_plan::rms_bwd_plan(rows, cols, (int)sizeof(T), vec, dw != nullptr);
+  const ts_plan::RmsNarrowPlan narrow =
+      ts_plan::rms_bwd_narrow_plan(rows, plan.reg ? nvec : 0);
+  if (narrow.tpr != 0) plan.nparts = dw != nullptr ? narrow.grid : 0;
   if (dw != nullptr && (size_t)plan.nparts * (size_t)cols * sizeof(float) > ws_bytes)
     return ts_host::fail(TS_ERR_WORKSPACE, "rmsnorm_bwd: plan needs %lld partial rows",
                          (long long)plan.nparts);
-  if (plan.wave) {
+  if (narrow.tpr != 0) {
+    float* part = dw != nullptr ? ws : nullptr;
+    bool launched = false;
+#define TS_LAUNCH_NARROW(TPR)                                                                  \
+  if (narrow.tpr == TPR) {                                                                     \
+    hipLaunchKernelGGL((rms_bwd_narrow<T, W, TPR>), dim3((unsigned)narrow.grid),               \
+                       dim3(ts_plan::kNarrowBlock), 0, st, dyp, lddy, xp, ldx, wp, rstd, dxp,  \
+                       lddx, part, rows, narrow.steps, (int)nvec, (float)cols);                \
+    launched = true;                                                                           \
+  }
+    TS_LAUNCH_NARROW(8)
+    TS_LAUNCH_NARROW(16)
+    TS_LAUNCH_NARROW(32)
+    TS_LAUNCH_NARROW(64)
+#undef TS_LAUNCH_NARROW
+    if (!launched)
+      return ts_host::fail(TS_ERR_INVALID_ARGUMENT, "rmsnorm_bwd: bad narrow plan (tpr=%d)",
+                           narrow.tpr);
+    ts_status s = ts_host::check_launch("rms_bwd_narrow");
+    if (s != TS_OK) return s;
+  } else if (plan.wave) {
     float* part = dw != nullptr ? ws : nullptr;
     bool launched = false;
 #define TS_LAUNCH_WAVE(KV)                                                                     \
@@ -744,7 +895,6 @@ ts_status bwd_typed(const void* dy, int64_t lddy, const void* x, int64_t ldx, co
                        (int)nvec, (float)cols);                                                 \
     launched = true;                                                                            \
   }
-    TS_LAUNCH_BWD(64, 1)
     TS_LAUNCH_BWD(128, 1)
     TS_LAUNCH_BWD(256, 1)
     TS_LAUNCH_BWD(512, 1)
