@@ -103,35 +103,48 @@ struct GemmArgs {
   LogitXform xf;
 };
 
-// Writes the wave's RW x 128 accumulator block (RW = 32 * kTI), rounded to
-// bf16, into its private LDS region as [row][col] with 256-byte rows.
+// Writes the wave's RW x 128 accumulator block (RW = 16 * kTI), rounded to
+// bf16, into its private LDS region as [row][col] with 256-byte rows. The four
+// 16-lane groups of a store hold rows 4 apart, whose 256-byte rows share the
+// banks: the bytes are XOR-swizzled by the row group in 32-byte units.
 template <int kTI>
 __device__ inline void stage_bf16(const Acc<kTI>& acc, uint8_t* region, int lane) {
+  const int g = lane >> 4;
 #pragma unroll
   for (int i = 0; i < kTI; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
+    for (int j = 0; j < 8; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const int row = i * 32 + 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-        const int col = j * 32 + (lane & 31);
-        *reinterpret_cast<__bf16*>(region + row * kStagePitch + col * 2) = (__bf16)acc.t[i][j][e];
+      for (int e = 0; e < 4; ++e) {
+        const int row = i * 16 + 4 * g + e;
+        const int byte = (j * 32 + (lane & 15) * 2) ^ (g << 5);
+        *reinterpret_cast<__bf16*>(region + row * kStagePitch + byte) = (__bf16)acc.t[i][j][e];
       }
 }
+// LDS byte offset of 16-byte chunk c of staged bf16 row `row`.
+__device__ inline int staged_chunk(int row, int c) {
+  return row * kStagePitch + ((c << 4) ^ (((row >> 2) & 3) << 5));
+}
 
-// Writes rows [32 i, 32 i + 32) of the wave's fp32 accumulator block (tile
-// row i) into its private LDS region as [row][col] fp32 with 512-byte rows
-// (16 KiB).
+// Writes rows [32 i, 32 i + 32) of the wave's fp32 accumulator block into its private LDS
+// region as [row][col] fp32 with 512-byte rows (16 KiB).
 template <int kTI>
 __device__ inline void stage_f32_tile(const Acc<kTI>& acc, int i, uint8_t* region, int lane) {
+  const int g = lane >> 4;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int h = 0; h < 2; ++h)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) {
-      const int row = 8 * (e >> 2) + 4 * (lane >> 5) + (e & 3);
-      const int col = j * 32 + (lane & 31);
-      *reinterpret_cast<float*>(region + row * 512 + col * 4) = acc.t[i][j][e];
-    }
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int row = h * 16 + 4 * g + e;
+        const int byte = (j * 64 + (lane & 15) * 4) ^ (g << 6);
+        *reinterpret_cast<float*>(region + row * 512 + byte) = acc.t[2 * i + h][j][e];
+      }
+}
+// LDS byte offset of byte b (a multiple of 16) of staged fp32 row `row`.
+__device__ inline int staged_f32(int row, int b) {
+  return row * 512 + (b ^ (((row >> 2) & 3) << 6));
 }
 
 // One 256 x 256 tile of C = A B^T with kW waves (ts_gemm::Cfg) and the
@@ -180,9 +193,8 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
   const int64_t mb = m0 + wm * Cw::RW;  // first row of this wave's block
   const int64_t nb = n0 + wn * 128;     // first column
   // Every wave is done with the pipeline's LDS before it is reused. Each wave
-  // then works in its own region (kLdsBytes / kW: 32 KiB with 4 waves, 16 KiB
-  // with 8); LDS operations of one wave complete in order, so it reads back
-  // its own writes without a barrier.
+  // then works in its own region (kLdsBytes / kW, 20 KiB); LDS operations of one
+  // wave complete in order, so it reads back its own writes without a barrier.
   constexpr int kRegion = (int)(ts_gemm::kLdsBytes / kW);
   static_assert(kRegion >= Cw::RW * kStagePitch && kRegion >= 32 * 512, "epilogue region");
   __syncthreads();
@@ -198,7 +210,7 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
     const int c8 = lane & 15;
     const int64_t gc = nb + c8 * 8;
 #pragma unroll
-    for (int i = 0; i < kTI; ++i) {
+    for (int i = 0; i < Cw::RW / 32; ++i) {
       const int64_t gm0 = mb + i * 32 + (lane >> 4);  // this lane's row at step s: gm0 + 4 s
       u32x4 old[8];
 #pragma unroll
@@ -213,8 +225,8 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
         const int lrow = 4 * s + (lane >> 4);
         const int64_t gm = gm0 + 4 * s;
         if (gm < a.M && gc < a.N) {
-          const float4 v0 = *reinterpret_cast<const float4*>(region + lrow * 512 + c8 * 32);
-          const float4 v1 = *reinterpret_cast<const float4*>(region + lrow * 512 + c8 * 32 + 16);
+          const float4 v0 = *reinterpret_cast<const float4*>(region + staged_f32(lrow, c8 * 32));
+          const float4 v1 = *reinterpret_cast<const float4*>(region + staged_f32(lrow, c8 * 32 + 16));
           float f[8];
           Elt<__bf16>::unpack(old[s], f);
           f[0] += v0.x;
@@ -240,7 +252,7 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
     constexpr bool kAddOld = kMode == kEpiAccF32 || kMode == kEpiAccBf16;
     constexpr int kPre = kAddOld ? 8 : 16;
 #pragma unroll
-    for (int i = 0; i < kTI; ++i) {
+    for (int i = 0; i < Cw::RW / 32; ++i) {
       const int64_t gm0 = mb + i * 32 + (lane >> 5);  // this lane's row at step it: gm0 + 2 it
 #pragma unroll
       for (int h = 0; h < 16; h += kPre) {
@@ -261,7 +273,7 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
           const int lrow = it * 2 + (lane >> 5);
           const int64_t gm = gm0 + 2 * it;
           if (gm < a.M && gc < a.N) {
-            float4 v = *reinterpret_cast<const float4*>(region + lrow * 512 + c4 * 16);
+            float4 v = *reinterpret_cast<const float4*>(region + staged_f32(lrow, c4 * 16));
             if constexpr (kAddOld) {
               const float4 o = old[q];
               v.x += o.x;
@@ -310,7 +322,7 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
       const int lrow = it * 4 + (lane >> 4);
       const int64_t gm = mb + lrow;
       const int64_t gc = nb + c16 * 8;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(region + lrow * kStagePitch + c16 * 16);
+      const u32x4 v = *reinterpret_cast<const u32x4*>(region + staged_chunk(lrow, c16));
       // a chunk of 8 columns is stored whole when it starts inside C (rows of C are
       // padded to whole chunks: ldc >= round_up(N, 8)); nin of its columns are < N,
       // fewer than 8 only in the last chunk when N % 8 != 0
@@ -842,11 +854,7 @@ Layout layout(int64_t N, int64_t H, int64_t V, int64_t chunk, bool grads, bool a
   return l;
 }
 
-// The GEMMs run with 8 waves (two per SIMD): measured on MI355X at C5 against
-// the 4-wave layout, logits 7.59 vs 7.88 ms, grad_hidden 6.96 vs 7.12 ms,
-// grad_weight 6.93 vs 7.19 ms, bit-identical results. The matrix cores are busier
-// per clock (69-76% against 58-67%); the box's clock under this load drops to
-// 1.55-1.6 GHz from 1.75-1.85, which takes back part of the gain.
+// The GEMMs run with 8 waves, two per SIMD (gemm.hpp).
 int64_t gemm_pieces(const GemmArgs& a) {
   return ((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN) * (a.splits > 1 ? a.splits : 1);
 }
@@ -982,7 +990,7 @@ extern "C" ts_status ts_flce_fwd_bwd(const void* hidden, int64_t ldh, const void
   if (ldh < H || ldw < H || ldh % 8 != 0 || ldw % 8 != 0)
     return fail(TS_ERR_SHAPE, "flce: row strides must be >= H and multiples of 8");
   // Buffer offsets are 32-bit and must stay below 2^31: within a 256-row K-major tile
-  // (row * ld * 2 bytes, ld = ldh, ldw or V) and within a 32-row k-block of an MN-major
+  // (row * ld * 2 bytes, ld = ldh, ldw or V) and within a 64-row k-block of an MN-major
   // operand (k * ld * 2, ld = ldh, ldw or V).
   if (V > ((int64_t)1 << 22) || H > ((int64_t)1 << 20) || N > ((int64_t)1 << 22))
     return fail(TS_ERR_SHAPE, "flce: shape beyond the kernel's index range");
@@ -1173,7 +1181,7 @@ ts_status check_two_pass(const char* who, const void* hidden, int64_t ldh, const
     return fail(TS_ERR_SHAPE, "%s: H must be a multiple of 8 (H=%lld)", who, (long long)H);
   if (ldh < H || ldw < H || ldh % 8 != 0 || ldw % 8 != 0)
     return fail(TS_ERR_SHAPE, "%s: row strides must be >= H and multiples of 8", who);
-  // 32-bit buffer offsets within a 256-row K-major tile and a 32-row MN-major k-block
+  // 32-bit buffer offsets within a 256-row K-major tile and a 64-row MN-major k-block
   if (V > ((int64_t)1 << 22) || H > ((int64_t)1 << 20) || N > ((int64_t)1 << 24) ||
       ldh > ((int64_t)1 << 22) || ldw > ((int64_t)1 << 22))
     return fail(TS_ERR_SHAPE, "%s: shape beyond the kernel's index range", who);

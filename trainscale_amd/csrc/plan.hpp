@@ -315,20 +315,20 @@ TS_HOST_DEVICE inline void gemm_tile_of(int64_t bid, int64_t MT, int64_t NT, int
 
 // K split of the linear-CE's grad_hidden GEMM, [M, K] @ [K, H] with K the vocabulary (or
 // one chunk of it). Its M x H tiles are few while K is long: at M = 1024, H = 768,
-// K = 50257 it has 12 tiles of 1571 k-blocks each, and 12 CUs work while the others have
+// K = 50257 it has 12 tiles of 786 k-blocks each, and 12 CUs work while the others have
 // long finished grad_weight's short tiles. So K is cut into `splits` slots, as many as
 // keep the pieces within one per CU (the grad_weight tiles of the same grid fill what is
 // left), each at least kSplitMinBlocks k-blocks long: a piece writes its fp32 partial
-// tile (256 KB, the time of about 10 k-blocks at a CU's share of HBM), and a second
+// tile (256 KB, the time of about 5 k-blocks at a CU's share of HBM), and a second
 // kernel sums the slots in order and rounds once. With a tile for every CU or more there
 // is one slot and nothing changes. The rule looks at M, H and K only, so every schedule
 // sums a given shape in the same order. Measured on MI355X, the gradient GEMMs of the shape
 // above: 1036 us whole, 174 us plus 11.5 us for the sum in 21 slots; of M = 2000, H = 4096,
 // K = 16128 (128 tiles): 566 us in two launches, 447 us in one grid with 2 slots.
 constexpr int64_t kGemmTile = 256;        // M and N of a tile
-constexpr int64_t kGemmBlockK = 32;       // a k-block
+constexpr int64_t kGemmBlockK = 64;       // a k-block
 constexpr int64_t kCus = 256;
-constexpr int64_t kSplitMinBlocks = 64;
+constexpr int64_t kSplitMinBlocks = 32;
 struct KSplit {
   int64_t splits;  // slots, at least 1
   int64_t kper;    // k per slot, whole k-blocks (the last slot may have fewer, or none)
