@@ -27,9 +27,12 @@
 // LDS rows of a K-major tile are 128 B (64 bf16) with the eight 16-byte chunks XOR-swizzled by
 // (row >> 1) & 7 (see swz), which makes the MFMA operand ds_read_b128s free of bank conflicts.
 //
-// MFMA 16x16x32 bf16 lane layout: A lane l holds row l % 16, k = (l / 16) * 8 + e for e < 8;
-// B lane l holds column l % 16 with the same k; accumulator element e is
-// C[4 * (l / 16) + e][l % 16].
+// MFMA 16x16x32 bf16 lane layout: the first operand's lane l holds row l % 16,
+// k = (l / 16) * 8 + e for e < 8; the second's lane l column l % 16 with the same k;
+// accumulator element e is D[4 * (l / 16) + e][l % 16]. B is passed first, so D is C
+// transposed and a lane holds, of each 16 x 16 tile of C, row l % 16 and the four consecutive
+// columns 4 * (l / 16) + e: an epilogue reads and writes C in 16-byte accesses straight from
+// the accumulators.
 //
 // Either operand may instead be stored MN-major (element (r, k) at k * ld + r,
 // e.g. dlogits [N, V] read as the [V, N] operand of the weight gradient, or
@@ -302,14 +305,15 @@ __device__ inline void read_op(const uint8_t* Xs, int r_base, int lane, int ks, 
 template <int kMajor>
 constexpr int frag_reads(int n) { return (kMajor == kMNMajor ? 2 : 1) * n; }
 
-// The MFMAs of a half step: every row tile against the four column tiles of `half`.
+// The MFMAs of a half step: every row tile against the four column tiles of `half`. B is the
+// first operand (see the layout of C above).
 template <int kTI>
 __device__ inline void mma_half(const bf16x8 (&a)[kTI], const bf16x8 (&b)[4], Acc<kTI>& acc,
                                 int half) {
 #pragma unroll
   for (int q = 0; q < kTI * 4; ++q)
     acc.t[q / 4][half * 4 + q % 4] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-        a[q / 4], b[q % 4], acc.t[q / 4][half * 4 + q % 4], 0, 0, 0);
+        b[q % 4], a[q / 4], acc.t[q / 4][half * 4 + q % 4], 0, 0, 0);
 }
 
 // Instruction interleaving. A wave issues MFMAs one at a time and waits for

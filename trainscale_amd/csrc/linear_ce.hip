@@ -37,8 +37,7 @@ using namespace ts;
 using ts_gemm::Acc;
 using ts_gemm::BM;
 using ts_gemm::BN;
-
-constexpr int kStagePitch = 256;  // bytes per staged epilogue row (128 bf16)
+using ts_gemm::f32x4;
 
 enum EpiMode : int {
   kEpiLogits = 0,     // bf16 C + row statistics
@@ -62,9 +61,7 @@ struct LogitXform {
   float inv_softcap;  // 1 / softcap
   float mul;
   __device__ inline bool on() const { return softcap > 0.f || mul != 1.f; }
-  __device__ inline float apply(float z) const {
-    return (softcap > 0.f ? softcap * tanhf(z * inv_softcap) : z) * mul;
-  }
+  __device__ inline float cap(float z) const { return softcap * tanhf(z * inv_softcap); }
   // t and dt/dz
   __device__ inline float apply_d(float z, float& dt) const {
     if (softcap > 0.f) {
@@ -103,48 +100,48 @@ struct GemmArgs {
   LogitXform xf;
 };
 
-// Writes the wave's RW x 128 accumulator block (RW = 16 * kTI), rounded to
-// bf16, into its private LDS region as [row][col] with 256-byte rows. The four
-// 16-lane groups of a store hold rows 4 apart, whose 256-byte rows share the
-// banks: the bytes are XOR-swizzled by the row group in 32-byte units.
-template <int kTI>
-__device__ inline void stage_bf16(const Acc<kTI>& acc, uint8_t* region, int lane) {
-  const int g = lane >> 4;
-#pragma unroll
-  for (int i = 0; i < kTI; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = i * 16 + 4 * g + e;
-        const int byte = (j * 32 + (lane & 15) * 2) ^ (g << 5);
-        *reinterpret_cast<__bf16*>(region + row * kStagePitch + byte) = (__bf16)acc.t[i][j][e];
-      }
+// Two bf16 roundings in one register, and back.
+__device__ inline uint32_t pack2(float lo, float hi) {
+  const bf16x2_t v = {(__bf16)lo, (__bf16)hi};
+  return __builtin_bit_cast(uint32_t, v);
 }
-// LDS byte offset of 16-byte chunk c of staged bf16 row `row`.
-__device__ inline int staged_chunk(int row, int c) {
-  return row * kStagePitch + ((c << 4) ^ (((row >> 2) & 3) << 5));
+__device__ inline float lo_f(uint32_t p) { return __builtin_bit_cast(float, p << 16); }
+__device__ inline float hi_f(uint32_t p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
+
+// Exchanges the odd 16-lane rows of x with the even ones of y.
+__device__ inline void swap_rows(uint32_t& x, uint32_t& y) {
+  typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));
+  const u32x2_t r =
+      __builtin_bit_cast(u32x2_t, __builtin_amdgcn_permlane16_swap(x, y, false, false));
+  x = r[0];
+  y = r[1];
 }
 
-// Writes rows [32 i, 32 i + 32) of the wave's fp32 accumulator block into its private LDS
-// region as [row][col] fp32 with 512-byte rows (16 KiB).
-template <int kTI>
-__device__ inline void stage_f32_tile(const Acc<kTI>& acc, int i, uint8_t* region, int lane) {
-  const int g = lane >> 4;
-#pragma unroll
-  for (int h = 0; h < 2; ++h)
-#pragma unroll
-    for (int j = 0; j < 8; ++j)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int row = h * 16 + 4 * g + e;
-        const int byte = (j * 64 + (lane & 15) * 4) ^ (g << 6);
-        *reinterpret_cast<float*>(region + row * 512 + byte) = acc.t[2 * i + h][j][e];
-      }
+// Rows of the epilogue in registers. Of 16 x 16 tile j of a row block, lane l holds row
+// l % 16 and columns 16 j + 4 g + e (g = l / 16, e < 4), in bf16 two packed registers. Two
+// tiles of 8-byte pieces become one 16-byte piece of 8 consecutive columns by swapping lane
+// rows: afterwards lane group g holds columns 8 * (g / 2) .. + 8 of tile 2p + g % 2, and the
+// four groups of a row 64 consecutive bytes of C. The exchange is its own inverse.
+__device__ inline u32x4 widen(uint32_t x0, uint32_t x1, uint32_t y0, uint32_t y1) {
+  swap_rows(x0, y0);
+  swap_rows(x1, y1);
+  return u32x4{x0, x1, y0, y1};
 }
-// LDS byte offset of byte b (a multiple of 16) of staged fp32 row `row`.
-__device__ inline int staged_f32(int row, int b) {
-  return row * 512 + (b ^ (((row >> 2) & 3) << 6));
+// Column, within the wave's 128, of the piece p < 4 that lane group g holds after widen.
+__device__ inline int wide_col(int p, int g) { return (2 * p + (g & 1)) * 16 + (g >> 1) * 8; }
+
+// Maximum and sum over the four lanes that share a row (l % 16); every lane gets the result.
+__device__ inline float groups_max(float v) {
+  uint32_t x = __builtin_bit_cast(uint32_t, v), y = x;
+  swap_rows(x, y);
+  const float m = fmaxf(__builtin_bit_cast(float, x), __builtin_bit_cast(float, y));
+  return fmaxf(m, __shfl_xor(m, 32));
+}
+__device__ inline float groups_sum(float v) {
+  uint32_t x = __builtin_bit_cast(uint32_t, v), y = x;
+  swap_rows(x, y);
+  const float s = __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y);
+  return s + __shfl_xor(s, 32);
 }
 
 // One 256 x 256 tile of C = A B^T with kW waves (ts_gemm::Cfg) and the
@@ -192,226 +189,214 @@ __device__ inline void gemm_tile(const GemmArgs& a, int64_t bid, uint8_t* smem) 
   const int wn = wid & 1;
   const int64_t mb = m0 + wm * Cw::RW;  // first row of this wave's block
   const int64_t nb = n0 + wn * 128;     // first column
-  // Every wave is done with the pipeline's LDS before it is reused. Each wave
-  // then works in its own region (kLdsBytes / kW, 20 KiB); LDS operations of one
-  // wave complete in order, so it reads back its own writes without a barrier.
-  constexpr int kRegion = (int)(ts_gemm::kLdsBytes / kW);
-  static_assert(kRegion >= Cw::RW * kStagePitch && kRegion >= 32 * 512, "epilogue region");
-  __syncthreads();
-  uint8_t* region = smem + wid * kRegion;
+  // The epilogue works on the accumulators as the lanes hold them (see widen): no LDS. Rows
+  // of C are whole 16-byte vectors (8 bf16), and one is read or written whole when its first
+  // column is inside C. Through LDS (2-byte stores of each accumulator, a row's statistics
+  // folded over 16 lanes for every 8 columns) the epilogue was bound by VALU and LDS issue:
+  // about 16 us a tile with statistics, now 11. Measured on MI355X, logits and statistics of
+  // [1024, 768] x [50257, 768] 132 -> 112 us, of [2000, 4096] x [128256, 4096] 1.74 -> 1.64 ms.
+  const int g = lane >> 4;
+  const int64_t gm0 = mb + (lane & 15);  // this lane's row of row block i: gm0 + 16 i
 
   if constexpr (kMode == kEpiAddBf16) {
-    // bf16 running sum C = bf16(C + acc): a lane owns 8 consecutive columns (16 bytes of
-    // C) of a 128-column row, 16 lanes a row, 4 rows a step. All 8 steps' old values of a
-    // 32-row tile are loaded before that tile is staged, so their latency overlaps the
-    // staging; the loads and stores are 16 bytes wide (measured on MI355X at the C5
-    // chunk shape: the gradient pair 3.57-3.59 ms against 3.65 ms with 8-byte accesses,
-    // 32 lanes a row).
-    const int c8 = lane & 15;
-    const int64_t gc = nb + c8 * 8;
+    // bf16 running sum C = bf16(C + acc). All old values are loaded before the first is used.
+    u32x4 old[kTI][4];
 #pragma unroll
-    for (int i = 0; i < Cw::RW / 32; ++i) {
-      const int64_t gm0 = mb + i * 32 + (lane >> 4);  // this lane's row at step s: gm0 + 4 s
-      u32x4 old[8];
+    for (int i = 0; i < kTI; ++i)
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const int64_t gm = gm0 + 4 * s;
-        // N % 8 == 0: a lane's 8 columns are all in or all out
-        old[s] = gm < a.M && gc < a.N ? ld16(a.C + gm * a.ldc + gc) : u32x4{0u, 0u, 0u, 0u};
+      for (int p = 0; p < 4; ++p) {
+        const int64_t gm = gm0 + 16 * i, gc = nb + wide_col(p, g);
+        old[i][p] = gm < a.M && gc < a.N ? ld16(a.C + gm * a.ldc + gc) : u32x4{0u, 0u, 0u, 0u};
       }
-      stage_f32_tile(acc, i, region, lane);
 #pragma unroll
-      for (int s = 0; s < 8; ++s) {
-        const int lrow = 4 * s + (lane >> 4);
-        const int64_t gm = gm0 + 4 * s;
-        if (gm < a.M && gc < a.N) {
-          const float4 v0 = *reinterpret_cast<const float4*>(region + staged_f32(lrow, c8 * 32));
-          const float4 v1 = *reinterpret_cast<const float4*>(region + staged_f32(lrow, c8 * 32 + 16));
-          float f[8];
-          Elt<__bf16>::unpack(old[s], f);
-          f[0] += v0.x;
-          f[1] += v0.y;
-          f[2] += v0.z;
-          f[3] += v0.w;
-          f[4] += v1.x;
-          f[5] += v1.y;
-          f[6] += v1.z;
-          f[7] += v1.w;
-          st16(a.C + gm * a.ldc + gc, Elt<__bf16>::pack(f));
-        }
+    for (int i = 0; i < kTI; ++i)
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        const int64_t gm = gm0 + 16 * i, gc = nb + wide_col(p, g);
+        const u32x4 o = old[i][p];
+        const u32x4 n = widen(o[0], o[1], o[2], o[3]);  // back to the accumulators' layout
+        const f32x4 x = acc.t[i][2 * p], y = acc.t[i][2 * p + 1];
+        const u32x4 v = widen(pack2(lo_f(n[0]) + x[0], hi_f(n[0]) + x[1]),
+                              pack2(lo_f(n[1]) + x[2], hi_f(n[1]) + x[3]),
+                              pack2(lo_f(n[2]) + y[0], hi_f(n[2]) + y[1]),
+                              pack2(lo_f(n[3]) + y[2], hi_f(n[3]) + y[3]));
+        if (gm < a.M && gc < a.N) st16(a.C + gm * a.ldc + gc, v);
       }
-    }
   } else if constexpr (kMode == kEpiF32 || kMode == kEpiAccF32 || kMode == kEpiAccBf16) {
-    // fp32 C32 rows of 128 columns = 512 B: 32 lanes x 16 B per row, 2 rows per step.
-    // The modes that add to what C32 holds load the old values of 8 steps at a time
-    // (16-byte fp32 values; more would exceed the register budget), the first batch
-    // before the tile is staged, so the loads' latency overlaps the staging instead of
-    // stalling step after step.
-    const int c4 = lane & 31;
-    const int64_t gc = nb + c4 * 4;
-    constexpr bool kAddOld = kMode == kEpiAccF32 || kMode == kEpiAccBf16;
-    constexpr int kPre = kAddOld ? 8 : 16;
+    // fp32 C32: a lane's four columns of a tile are 16 bytes. In the modes that add to what
+    // C32 holds, the old values of the next row block are loaded while one is worked on.
+    constexpr bool kOld = kMode != kEpiF32;
+    f32x4 old[2][8];
+    auto load_old = [&](int i) {
+      const int64_t gm = gm0 + 16 * i;
 #pragma unroll
-    for (int i = 0; i < Cw::RW / 32; ++i) {
-      const int64_t gm0 = mb + i * 32 + (lane >> 5);  // this lane's row at step it: gm0 + 2 it
+      for (int j = 0; j < 8; ++j) {
+        const int64_t gc = nb + j * 16 + g * 4;
+        old[i & 1][j] = gm < a.M && gc < a.N
+                            ? *reinterpret_cast<const f32x4*>(C32 + gm * a.ldc32 + gc)
+                            : f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    };
+    if constexpr (kOld) load_old(0);
 #pragma unroll
-      for (int h = 0; h < 16; h += kPre) {
-        float4 old[kAddOld ? kPre : 1];
-        if constexpr (kAddOld) {
+    for (int i = 0; i < kTI; ++i) {
+      const int64_t gm = gm0 + 16 * i;
+      if constexpr (kOld) {
+        if (i + 1 < kTI) load_old(i + 1);
 #pragma unroll
-          for (int q = 0; q < kPre; ++q) {
-            const int64_t gm = gm0 + 2 * (h + q);
-            const bool in = gm < a.M && gc < a.N;  // N % 8 == 0: 4 columns all in or all out
-            old[q] = in ? *reinterpret_cast<const float4*>(C32 + gm * a.ldc32 + gc)
-                        : make_float4(0.f, 0.f, 0.f, 0.f);
-          }
+        for (int j = 0; j < 8; ++j) acc.t[i][j] += old[i & 1][j];
+      }
+      if constexpr (kMode == kEpiAccBf16) {
+#pragma unroll
+        for (int p = 0; p < 4; ++p) {
+          const f32x4 x = acc.t[i][2 * p], y = acc.t[i][2 * p + 1];
+          const u32x4 v =
+              widen(pack2(x[0], x[1]), pack2(x[2], x[3]), pack2(y[0], y[1]), pack2(y[2], y[3]));
+          const int64_t gc = nb + wide_col(p, g);
+          if (gm < a.M && gc < a.N) st16(a.C + gm * a.ldc + gc, v);
         }
-        if (h == 0) stage_f32_tile(acc, i, region, lane);
+      } else {
 #pragma unroll
-        for (int q = 0; q < kPre; ++q) {
-          const int it = h + q;
-          const int lrow = it * 2 + (lane >> 5);
-          const int64_t gm = gm0 + 2 * it;
-          if (gm < a.M && gc < a.N) {
-            float4 v = *reinterpret_cast<const float4*>(region + staged_f32(lrow, c4 * 16));
-            if constexpr (kAddOld) {
-              const float4 o = old[q];
-              v.x += o.x;
-              v.y += o.y;
-              v.z += o.z;
-              v.w += o.w;
-            }
-            if constexpr (kMode == kEpiAccBf16) {
-              bf16x2_t lo = {(__bf16)v.x, (__bf16)v.y};
-              bf16x2_t hi = {(__bf16)v.z, (__bf16)v.w};
-              uint2 pk;
-              pk.x = __builtin_bit_cast(uint32_t, lo);
-              pk.y = __builtin_bit_cast(uint32_t, hi);
-              *reinterpret_cast<uint2*>(a.C + gm * a.ldc + gc) = pk;
-            } else {
-              *reinterpret_cast<float4*>(C32 + gm * a.ldc32 + gc) = v;
-            }
-          }
+        for (int j = 0; j < 8; ++j) {
+          const int64_t gc = nb + j * 16 + g * 4;
+          if (gm < a.M && gc < a.N)
+            *reinterpret_cast<f32x4*>(C32 + gm * a.ldc32 + gc) = acc.t[i][j];
         }
       }
     }
   } else {
-    stage_bf16(acc, region, lane);
-    const int c16 = lane & 15;  // 16-byte chunk of the 256-byte row
-    const int64_t nparts = 2 * ((a.N + BN - 1) / BN);
-    // Row operands of the statistics and dlogits epilogues: lane i holds those
-    // of the wave's row mb + i; the 16 lanes that handle a row fetch them with
-    // ds_bpermute. rel_lab is the label's column in C, -1 when outside it.
-    int rel_lab = -1;
-    float lse2 = 0.f, dsc = 0.f;
+    const int64_t nparts = 2 * NT;
+    // columns of the wave's 128 that lie in C
+    const int ncols = a.N - nb < 128 ? (a.N > nb ? (int)(a.N - nb) : 0) : 128;
+    // Row operands: the label's column of the wave's 128 less this lane's first (a lane's
+    // columns are 16 j + e; -1 when the label is outside the wave's), lse and row scale.
+    int lab[kTI];
+    float l2[kTI], ds[kTI];
     if constexpr (kMode == kEpiStats || kMode == kEpiDlogits) {
-      static_assert(Cw::RW == 64, "one row per lane");
-      const int64_t r = mb + lane;
-      if (r < a.M) {
-        const int64_t c = a.labels[r] - a.label_offset;
-        rel_lab = c >= 0 && c < a.N ? (int)c : -1;
-        if constexpr (kMode == kEpiDlogits) {
-          lse2 = a.lse[r] * kLog2e;
-          dsc = a.dscale[r];
+#pragma unroll
+      for (int i = 0; i < kTI; ++i) {
+        const int64_t gm = gm0 + 16 * i;
+        lab[i] = -1;
+        l2[i] = ds[i] = 0.f;
+        if (gm < a.M) {
+          const int64_t c = a.labels[gm] - a.label_offset;
+          lab[i] = c >= nb && c < a.N && c - nb < 128 ? (int)(c - nb) - 4 * g : -1;
+          if constexpr (kMode == kEpiDlogits) {
+            l2[i] = a.lse[gm] * kLog2e;
+            ds[i] = a.dscale[gm];
+          }
         }
       }
     }
-    const bool xf_on = a.xf.on();
-#pragma unroll 4
-    for (int it = 0; it < Cw::RW / 4; ++it) {
-      const int lrow = it * 4 + (lane >> 4);
-      const int64_t gm = mb + lrow;
-      const int64_t gc = nb + c16 * 8;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(region + staged_chunk(lrow, c16));
-      // a chunk of 8 columns is stored whole when it starts inside C (rows of C are
-      // padded to whole chunks: ldc >= round_up(N, 8)); nin of its columns are < N,
-      // fewer than 8 only in the last chunk when N % 8 != 0
-      const bool in = gm < a.M && gc < a.N;
-      const int nin = in ? (a.N - gc < 8 ? (int)(a.N - gc) : 8) : 0;
-      if constexpr (kMode == kEpiLogits || kMode == kEpiBf16) {
-        if (in) st16(a.C + gm * a.ldc + gc, v);
+#pragma unroll
+    for (int i = 0; i < kTI; ++i) {
+      const int64_t gm = gm0 + 16 * i;
+      uint32_t pk[8][2];  // the row's bf16 logits
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        pk[j][0] = pack2(acc.t[i][j][0], acc.t[i][j][1]);
+        pk[j][1] = pack2(acc.t[i][j][2], acc.t[i][j][3]);
+      }
+      float f[8][4];
+      if constexpr (kMode != kEpiBf16) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          f[j][0] = lo_f(pk[j][0]);
+          f[j][1] = hi_f(pk[j][0]);
+          f[j][2] = lo_f(pk[j][1]);
+          f[j][3] = hi_f(pk[j][1]);
+        }
       }
       if constexpr (kMode == kEpiStats) {
-        // statistics of t over the row's 128-column slice, and t at the label; the
-        // logits themselves when the caller keeps them for the backward
-        if (in && a.C != nullptr) st16(a.C + gm * a.ldc + gc, v);
-        float f[8];
-        Elt<__bf16>::unpack(v, f);
-        if (xf_on) {
+        // uniform branches around whole loops: inside, they would split each value's code
+        if (a.xf.softcap > 0.f) {
 #pragma unroll
-          for (int q = 0; q < 8; ++q) f[q] = a.xf.apply(f[q]);
+          for (int q = 0; q < 32; ++q) f[q / 4][q % 4] = a.xf.cap(f[q / 4][q % 4]);
         }
-        if (nin < 8) {  // columns past N take no part in the statistics
+        if (a.xf.mul != 1.f) {
 #pragma unroll
-          for (int q = 0; q < 8; ++q) f[q] = q < nin ? f[q] : -INFINITY;
-        }
-        float lm = f[0];
-#pragma unroll
-        for (int q = 1; q < 8; ++q) lm = fmaxf(lm, f[q]);
-        const float m = row_max(in ? lm : -INFINITY);  // over the 16 lanes of this row
-        float ls = 0.f;
-        if (in) {
-          const float mb2 = m * kLog2e;
-#pragma unroll
-          for (int q = 0; q < 8; ++q) ls += fast_exp2(__builtin_fmaf(f[q], kLog2e, -mb2));
-        }
-        const float s = row_sum(ls);
-        if (gm < a.M && c16 == 0) a.stats[gm * nparts + nt * 2 + wn] = make_float2(m, s);
-        const int d = __shfl(rel_lab, lrow) - (int)gc;
-        if (in && (unsigned)d < 8u) {
-          float zl = f[0];
-#pragma unroll
-          for (int q = 1; q < 8; ++q) zl = d == q ? f[q] : zl;
-          a.zlab[gm] = zl;
+          for (int q = 0; q < 32; ++q) f[q / 4][q % 4] *= a.xf.mul;
         }
       }
       if constexpr (kMode == kEpiDlogits) {
-        // (exp(t - lse) - onehot) * dt/dz * dscale, rounded to bf16
-        const float l2 = __shfl(lse2, lrow);
-        const float ds = __shfl(dsc, lrow);
-        const int d = __shfl(rel_lab, lrow) - (int)gc;
-        float f[8], g[8];
-        Elt<__bf16>::unpack(v, f);
-        if (!xf_on) {
+        // (exp(t - lse) - onehot) * dt/dz * dscale, rounded to bf16; dt/dz is one factor of
+        // the row without a softcap
+        float dt[8][4];
+        if (a.xf.softcap > 0.f) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float pr = fast_exp2(__builtin_fmaf(f[e], kLog2e, -l2));
-            g[e] = ds * (e == d ? pr - 1.f : pr);
-          }
+          for (int q = 0; q < 32; ++q)
+            f[q / 4][q % 4] = a.xf.apply_d(f[q / 4][q % 4], dt[q / 4][q % 4]);
         } else {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            float dt;
-            const float t = a.xf.apply_d(f[e], dt);
-            const float pr = fast_exp2(__builtin_fmaf(t, kLog2e, -l2));
-            g[e] = ds * (e == d ? pr - 1.f : pr) * dt;
-          }
+          for (int q = 0; q < 32; ++q) f[q / 4][q % 4] *= a.xf.mul;
         }
-        if (nin < 8) {  // columns past N: zero, the gradient GEMMs read them
 #pragma unroll
-          for (int e = 0; e < 8; ++e) g[e] = e < nin ? g[e] : 0.f;
+        for (int q = 0; q < 32; ++q)
+          f[q / 4][q % 4] = fast_exp2(__builtin_fmaf(f[q / 4][q % 4], kLog2e, -l2[i]));
+        if (lab[i] >= 0 && (lab[i] & 15) < 4) {
+#pragma unroll
+          for (int q = 0; q < 32; ++q)
+            f[q / 4][q % 4] -= lab[i] == (q / 4) * 16 + q % 4 ? 1.f : 0.f;
         }
-        if (in) st16(a.C + gm * a.ldc + gc, Elt<__bf16>::pack(g));
+        if (a.xf.softcap > 0.f) {
+#pragma unroll
+          for (int q = 0; q < 32; ++q) f[q / 4][q % 4] = ds[i] * f[q / 4][q % 4] * dt[q / 4][q % 4];
+        } else {
+#pragma unroll
+          for (int q = 0; q < 32; ++q) f[q / 4][q % 4] = ds[i] * f[q / 4][q % 4] * a.xf.mul;
+        }
+        if (ncols < 128) {  // columns past N: zero, the gradient GEMMs read them
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[j][e] = 16 * j + 4 * g + e < ncols ? f[j][e] : 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          pk[j][0] = pack2(f[j][0], f[j][1]);
+          pk[j][1] = pack2(f[j][2], f[j][3]);
+        }
       }
-      if constexpr (kMode == kEpiLogits) {
-        float f[8];
-        Elt<__bf16>::unpack(v, f);
-        if (nin < 8) {  // columns past N take no part in the statistics
+      if (kMode != kEpiStats || a.C != nullptr) {
 #pragma unroll
-          for (int q = 0; q < 8; ++q) f[q] = q < nin ? f[q] : -INFINITY;
+        for (int p = 0; p < 4; ++p) {
+          const u32x4 v = widen(pk[2 * p][0], pk[2 * p][1], pk[2 * p + 1][0], pk[2 * p + 1][1]);
+          const int col = wide_col(p, g);
+          if (gm < a.M && col < ncols) st16(a.C + gm * a.ldc + nb + col, v);
         }
-        float lm = f[0];
+      }
+      if constexpr (kMode == kEpiLogits || kMode == kEpiStats) {
+        // Statistics over the row's 128-column slice: a lane folds its 32 columns, then the
+        // four lanes of the row are combined.
+        if (ncols < 128) {  // columns past N take no part
 #pragma unroll
-        for (int q = 1; q < 8; ++q) lm = fmaxf(lm, f[q]);
-        const float m = row_max(in ? lm : -INFINITY);  // over the 16 lanes of this row
-        float ls = 0.f;
-        if (in) {
-          const float mb = m * kLog2e;
+          for (int j = 0; j < 8; ++j)
 #pragma unroll
-          for (int q = 0; q < 8; ++q) ls += fast_exp2(__builtin_fmaf(f[q], kLog2e, -mb));
+            for (int e = 0; e < 4; ++e)
+              f[j][e] = 16 * j + 4 * g + e < ncols ? f[j][e] : -INFINITY;
         }
-        const float s = row_sum(ls);
-        if (gm < a.M && c16 == 0) a.stats[gm * nparts + nt * 2 + wn] = make_float2(m, s);
+        float lm = f[0][0];
+#pragma unroll
+        for (int q = 1; q < 32; ++q) lm = fmaxf(lm, f[q / 4][q % 4]);
+        const float m = groups_max(lm);
+        const float m2 = m * kLog2e;
+        float ls[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) ls[e] += fast_exp2(__builtin_fmaf(f[j][e], kLog2e, -m2));
+        float s = groups_sum((ls[0] + ls[1]) + (ls[2] + ls[3]));
+        if (ncols == 0) s = 0.f;  // a slice past N (uniform)
+        if (gm < a.M && g == 0) a.stats[gm * nparts + nt * 2 + wn] = make_float2(m, s);
+      }
+      if constexpr (kMode == kEpiStats) {
+        // t at the label, where this lane holds its column
+        if (lab[i] >= 0 && (lab[i] & 15) < 4) {
+          float zl = f[0][0];
+#pragma unroll
+          for (int q = 1; q < 32; ++q) zl = lab[i] == (q / 4) * 16 + q % 4 ? f[q / 4][q % 4] : zl;
+          a.zlab[gm] = zl;
+        }
       }
     }
   }
