@@ -497,11 +497,13 @@ ts_status ts_flce_forward(const void* hidden, int64_t ldh, const void* weight, i
  *   dz = bf16(dt * dt/dz),  grad_hidden = dz @ weight,  grad_weight = dz^T @ hidden
  * (bf16 outputs, fp32 accumulation; either may be NULL). lse: the forward's.
  * The logits are recomputed one vocabulary chunk of chunk_cols columns at a
- * time (0: about V / 8, at least 4096; rounded up to 256) by the forward's
+ * time (0: about V / 8, at least 4096 and at least what keeps N x chunk at 256
+ * MB of dz; rounded up to 256) by the forward's
  * GEMM, whose epilogue forms the chunk's dz; grad_hidden accumulates over the
  * chunks in fp32, grad_weight's rows of a chunk are written once. Workspace:
  * ts_flce_backward_workspace_size(N, H, V, chunk_cols) bytes (N x chunk bf16
- * dz, plus N x H fp32 with more than one chunk). Deterministic.
+ * dz, plus N x H fp32 with more than one chunk, or N x H fp32 for each K slot
+ * where grad_hidden's product is cut along K: at most 64 MB). Deterministic.
  * Replaces autograd's backward through chunked_log_softmax /
  * selective_log_softmax (rl_training.py:95-191) and the lm_head matmul.
  */

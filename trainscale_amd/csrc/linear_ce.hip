@@ -1117,12 +1117,23 @@ FwdLayout fwd_layout(int64_t N, int64_t V) {
   return l;
 }
 
-// Vocabulary chunk of the backward: the given width rounded up to whole
-// 256-column tiles, or the default, about an eighth of V (at least 4096
-// columns), so the dlogits buffer holds N x chunk bf16 values.
-int64_t bwd_chunk_cols(int64_t V, int64_t chunk_cols) {
-  int64_t c = chunk_cols > 0 ? chunk_cols : ((V + 7) / 8 + BN - 1) / BN * BN;
-  if (chunk_cols <= 0 && c < 4096) c = 4096;
+// Vocabulary chunk of the backward: the given width rounded up to whole 256-column tiles, or
+// the default: about an eighth of V, and at least as many columns as keep the N x chunk bf16
+// dlogits at kBwdChunkBytes (and at least 4096). Few tokens make narrow chunks' GEMMs short
+// of tiles and each chunk costs its launches; with the scratch that large batches take
+// anyway they need few chunks or one. Measured on MI355X, the backward with chunks of V / 8
+// (at least 4096 columns) against this rule: 1000 tokens, H = 1024, V = 32000 662 -> 205 us;
+// 100, 768, 50257 566 -> 87 us; 400, 4096, 128256 1.86 -> 1.45 ms; 4096, 2048, 50257
+// 2.32 -> 2.20 ms; 2000 or 8192, 4096, 128256 within 1%, whatever the chunk.
+constexpr int64_t kBwdChunkBytes = (int64_t)256 << 20;
+int64_t bwd_chunk_cols(int64_t N, int64_t V, int64_t chunk_cols) {
+  int64_t c = chunk_cols;
+  if (chunk_cols <= 0) {
+    c = (V + 7) / 8;
+    const int64_t fit = kBwdChunkBytes / 2 / N / BN * BN;
+    if (c < fit) c = fit;
+    if (c < 4096) c = 4096;
+  }
   c = (c + BN - 1) / BN * BN;
   const int64_t v8 = (V + 7) / 8 * 8;
   return c > v8 ? v8 : c;
@@ -1136,7 +1147,7 @@ struct BwdLayout {
 
 BwdLayout bwd_layout(int64_t N, int64_t H, int64_t V, int64_t chunk_cols) {
   BwdLayout l{};
-  l.chunk = bwd_chunk_cols(V, chunk_cols);
+  l.chunk = bwd_chunk_cols(N, V, chunk_cols);
   l.nchunks = (V + l.chunk - 1) / l.chunk;
   l.splits = ts_plan::hidden_split(N, H, l.chunk < V ? l.chunk : V).splits;
   size_t off = 0;

@@ -55,13 +55,19 @@ __all__ = ["LinearCrossEntropyFunction", "FusedLinearCrossEntropyFunction",
            "linear_ce_forward", "linear_ce_backward", "linear_ce_forward_backward",
            "VocabShardState", "linear_ce_vocab_phase1", "linear_ce_vocab_phase2"]
 
-# The one-call schedule's token chunk with chunk_tokens=None: half the tokens
-# (rounded up to 256 rows), so its bf16 logits scratch stays within half of the
-# [N, V] logits; batches of up to 256 tokens run as one chunk. Measured on MI355X
-# at C5 (N = 8192): 21.5 ms with two chunks of 4096 tokens, 22.5 ms with four of
-# 2048 (two more bf16 read-modify-write passes over grad_weight), 21.4 ms with all
-# the logits in one chunk.
+# The one-call schedule's token chunk with chunk_tokens=None: all the tokens while their
+# bf16 logits take at most _ONE_CHUNK_BYTES (and up to 256 tokens in any case), else half
+# the tokens (rounded up to 256 rows), so larger batches' scratch stays within half of the
+# [N, V] logits. One chunk reads the LM head once and rounds grad_weight once; the bound is
+# the scratch that half of C5's tokens take (N = 8192: 1.05 GB). Measured on MI355X,
+# two chunks against one: N = 512, H = 4096, V = 128256 2.27 -> 1.60 ms; 2048 tokens
+# 5.78 -> 5.19; 4096 tokens 10.6 -> 10.0; 2045, 768, 50257 726 -> 615 us; at C5, above
+# the bound, 20.08 and 19.77 ms (and 22.5 against 21.5 with four chunks and two). Vocabularies
+# smaller than any LM head's (below 4096 columns) keep the two chunks: nothing is gained there
+# but launches, and small inputs keep running the sum over chunks.
 DEFAULT_TOKEN_CHUNKS = 2
+_ONE_CHUNK_BYTES = 1 << 30
+_ONE_CHUNK_MIN_V = 4096
 
 _REDUCTIONS = {"mean": 0, "sum": 1}
 TS_FLCE_GRADS, TS_FLCE_ACCUM_BF16 = 1, 2  # include/trainscale_amd.h
@@ -69,9 +75,12 @@ _REDUCTIONS_2P = {"mean": 0, "sum": 1, "none": 2}
 
 
 def _chunk_rows(N: int, V: int, chunk_tokens: Optional[int]) -> int:
-    """Token chunk of the one-call schedule (0: one chunk)."""
+    """Token chunk of the one-call schedule (0: one chunk): chunk_tokens, or by default one
+    chunk while the bf16 logits take at most _ONE_CHUNK_BYTES, else half the tokens."""
     if chunk_tokens is not None:
         return int(chunk_tokens)
+    if V >= _ONE_CHUNK_MIN_V and N * _logits_ld(V) * 2 <= _ONE_CHUNK_BYTES:
+        return 0
     rows = -(-N // DEFAULT_TOKEN_CHUNKS)
     rows = -(-rows // 256) * 256
     return 0 if rows >= N else rows
@@ -165,7 +174,7 @@ def linear_ce_backward(hidden: Tensor, weight: Tensor, labels: Tensor, lse: Tens
     """ts_flce_backward: (grad_hidden [N, H] or None, grad_weight [V, H] or None) for the
     upstream gradient dloss (one value for mean/sum, or [N] per-row values for "none";
     a single value broadcasts). vocab_chunk: columns per recomputed chunk (default
-    about V/8). With `logits`, the [N, V] bf16 logits linear_ce_forward kept
+    about V/8, or as many as keep the chunk's dlogits at 256 MB). With `logits`, the [N, V] bf16 logits linear_ce_forward kept
     (keep_logits), ts_flce_backward_kept forms the gradients from them instead of
     recomputing, and overwrites them."""
     if reduction not in _REDUCTIONS_2P:
@@ -218,7 +227,7 @@ def linear_ce_forward_backward(hidden: Tensor, weight: Tensor, labels: Tensor,
                                grad_weight_accum: str = "fp32"):
     """Runs ts_flce_fwd_bwd; returns (loss fp32 0-d, loss_rows [N], lse [N],
     grad_hidden or None, grad_weight or None) for an upstream gradient of 1.
-    chunk_tokens: rows per token chunk (None: half the tokens, 0: one chunk);
+    chunk_tokens: rows per token chunk (None: see _chunk_rows, 0: one chunk);
     grad_weight_accum: "fp32" (a V x H fp32 workspace, rounded once) or "bf16" (summed
     in the bf16 output, rounded after each chunk)."""
     if grad_weight_accum not in ("fp32", "bf16"):
