@@ -424,14 +424,25 @@ void flce_gemm_pair(const GemmArgs a1, const GemmArgs a2, int64_t tiles1) {
   else gemm_tile<kMode2, kMA2, kMB2, kW>(a2, bid - tiles1, smem);
 }
 
-// n_valid = #labels != ignore_index over all N rows (one workgroup, fixed order).
-__global__ __launch_bounds__(256) void flce_count(const int64_t* __restrict__ labels, int64_t N,
-                                                  int64_t ignore_index, int* __restrict__ n_valid) {
-  __shared__ float red[4];
+// The single-workgroup kernels over all rows: a chain of dependent-latency steps, so as many
+// threads as a workgroup has (N = 8192 on MI355X: 15 us with 256 threads, 5 with 1024).
+constexpr int kOneWg = 1024;
+
+// n_valid = #labels != ignore_index over all N rows (one workgroup, fixed order), and, where
+// scale is not NULL, the loss scale: 1 / max(n_valid, 1) for the mean, else 1.
+__global__ __launch_bounds__(kOneWg) void flce_count(const int64_t* __restrict__ labels, int64_t N,
+                                                     int64_t ignore_index,
+                                                     int* __restrict__ n_valid, int mean,
+                                                     float* __restrict__ scale) {
+  __shared__ float red[kOneWg / 64];
   float c = 0.f;
-  for (int64_t i = threadIdx.x; i < N; i += 256) c += labels[i] != ignore_index ? 1.f : 0.f;
-  c = block_sum<4>(c, red);
-  if (threadIdx.x == 0) *n_valid = (int)c;
+#pragma unroll 4
+  for (int64_t i = threadIdx.x; i < N; i += kOneWg) c += labels[i] != ignore_index ? 1.f : 0.f;
+  c = block_sum<kOneWg / 64>(c, red);
+  if (threadIdx.x != 0) return;
+  const int n = (int)c;
+  *n_valid = n;
+  if (scale != nullptr) *scale = mean ? 1.f / (float)(n > 0 ? n : 1) : 1.f;
 }
 
 // Row waves per workgroup of the one-wave-per-row kernels.
@@ -590,20 +601,16 @@ __global__ __launch_bounds__(64) void flce_vocab_merge(const ShardStats* __restr
 }
 
 // loss = scale * sum(loss_rows) over all N rows (one workgroup, fixed order);
-// scale = 1/max(n_valid, 1) for the mean, 1 for the sum. Also stores the scale.
-__global__ __launch_bounds__(256) void flce_loss(const float* __restrict__ loss_rows, int64_t N,
-                                                 const int* __restrict__ n_valid, int mean,
-                                                 float* __restrict__ loss,
-                                                 float* __restrict__ scale_out) {
-  __shared__ float red[4];
+// scale = 1/max(n_valid, 1) for the mean, 1 for the sum.
+__global__ __launch_bounds__(kOneWg) void flce_loss(const float* __restrict__ loss_rows, int64_t N,
+                                                    const int* __restrict__ n_valid, int mean,
+                                                    float* __restrict__ loss) {
+  __shared__ float red[kOneWg / 64];
   float s = 0.f;
-  for (int64_t i = threadIdx.x; i < N; i += 256) s += loss_rows[i];
-  s = block_sum<4>(s, red);
-  if (threadIdx.x == 0) {
-    const float scale = mean ? 1.f / (float)(*n_valid > 0 ? *n_valid : 1) : 1.f;
-    *loss = s * scale;
-    *scale_out = scale;
-  }
+#pragma unroll 4
+  for (int64_t i = threadIdx.x; i < N; i += kOneWg) s += loss_rows[i];
+  s = block_sum<kOneWg / 64>(s, red);
+  if (threadIdx.x == 0) *loss = s * (mean ? 1.f / (float)(*n_valid > 0 ? *n_valid : 1) : 1.f);
 }
 
 // dlogits of a chunk in place: D = (exp(z - lse) - onehot) * scale in bf16
@@ -1018,16 +1025,12 @@ extern "C" ts_status ts_flce_fwd_bwd(const void* hidden, int64_t ldh, const void
   const __bf16* Wd = static_cast<const __bf16*>(weight);
   const int64_t ldl = logits_ld(V);
 
-  hipLaunchKernelGGL(flce_count, dim3(1), dim3(256), 0, st, labels, N, ignore_index, n_valid);
+  hipLaunchKernelGGL(flce_count, dim3(1), dim3(kOneWg), 0, st, labels, N, ignore_index, n_valid,
+                     reduction == 0 ? 1 : 0, scale);
   TS_TRY(ts_host::check_launch("flce_count"));
   // Pass 1 over chunks: logits, statistics, per-row loss (and lse).
   // With gradients the dlogits of a chunk are consumed right away, so the
-  // loss scale (which needs every row's label) is computed up front.
-  if (grads) {
-    hipLaunchKernelGGL(flce_loss, dim3(1), dim3(256), 0, st, rows_ws, (int64_t)0, n_valid,
-                       reduction == 0 ? 1 : 0, loss, scale);
-    TS_TRY(ts_host::check_launch("flce_loss"));
-  }
+  // loss scale (which needs every row's label) is computed up front, with the count.
   for (int64_t c = 0; c < lay.nchunks; ++c) {
     const int64_t r0 = c * lay.chunk;
     const int64_t Mc = N - r0 < lay.chunk ? N - r0 : lay.chunk;
@@ -1083,8 +1086,8 @@ extern "C" ts_status ts_flce_fwd_bwd(const void* hidden, int64_t ldh, const void
                                             : kEpiAccBf16;
     TS_TRY(launch_grads_full_k(dh, dw, wmode, part, st, "flce_gemm_grads"));
   }
-  hipLaunchKernelGGL(flce_loss, dim3(1), dim3(256), 0, st, rows_ws, N, n_valid,
-                     reduction == 0 ? 1 : 0, loss, scale);
+  hipLaunchKernelGGL(flce_loss, dim3(1), dim3(kOneWg), 0, st, rows_ws, N, n_valid,
+                     reduction == 0 ? 1 : 0, loss);
   return ts_host::check_launch("flce_loss");
 }
 
@@ -1236,7 +1239,6 @@ ts_status flce_forward_impl(const char* who, const void* hidden, int64_t ldh, co
   float* rows_ws = loss_rows != nullptr ? loss_rows : reinterpret_cast<float*>(ws + lay.off_rows);
   float* lse_ws = lse != nullptr ? lse : reinterpret_cast<float*>(ws + lay.off_lse);
   int* n_valid = reinterpret_cast<int*>(ws + lay.off_misc);
-  float* sc = reinterpret_cast<float*>(ws + lay.off_misc + 16);
   GemmArgs g{};
   g.A = static_cast<const __bf16*>(hidden);
   g.lda = ldh;
@@ -1257,10 +1259,11 @@ ts_status flce_forward_impl(const char* who, const void* hidden, int64_t ldh, co
                      lay.nparts, zlab, labels, N, V, ignore_index, lse_ws, rows_ws);
   TS_TRY(ts_host::check_launch("flce_rows_t"));
   if (loss == nullptr) return TS_OK;
-  hipLaunchKernelGGL(flce_count, dim3(1), dim3(256), 0, st, labels, N, ignore_index, n_valid);
+  hipLaunchKernelGGL(flce_count, dim3(1), dim3(kOneWg), 0, st, labels, N, ignore_index, n_valid, 0,
+                     static_cast<float*>(nullptr));
   TS_TRY(ts_host::check_launch("flce_count"));
-  hipLaunchKernelGGL(flce_loss, dim3(1), dim3(256), 0, st, rows_ws, N, n_valid,
-                     reduction == 0 ? 1 : 0, loss, sc);
+  hipLaunchKernelGGL(flce_loss, dim3(1), dim3(kOneWg), 0, st, rows_ws, N, n_valid,
+                     reduction == 0 ? 1 : 0, loss);
   return ts_host::check_launch("flce_loss");
 }
 
@@ -1340,7 +1343,8 @@ extern "C" ts_status ts_flce_backward(const void* hidden, int64_t ldh, const voi
   const __bf16* Hd = static_cast<const __bf16*>(hidden);
   const __bf16* Wd = static_cast<const __bf16*>(weight);
 
-  hipLaunchKernelGGL(flce_count, dim3(1), dim3(256), 0, st, labels, N, ignore_index, n_valid);
+  hipLaunchKernelGGL(flce_count, dim3(1), dim3(kOneWg), 0, st, labels, N, ignore_index, n_valid, 0,
+                     static_cast<float*>(nullptr));
   TS_TRY(ts_host::check_launch("flce_count"));
   hipLaunchKernelGGL(flce_dscale, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, labels, N,
                      ignore_index, dloss, dloss_stride, n_valid, reduction == 0 ? 1 : 0, dscale);
@@ -1482,7 +1486,8 @@ extern "C" ts_status ts_flce_backward_kept(const void* hidden, int64_t ldh, cons
   int* n_valid = reinterpret_cast<int*>(ws + lay.off_misc);
   __bf16* L = static_cast<__bf16*>(logits);
 
-  hipLaunchKernelGGL(flce_count, dim3(1), dim3(256), 0, st, labels, N, ignore_index, n_valid);
+  hipLaunchKernelGGL(flce_count, dim3(1), dim3(kOneWg), 0, st, labels, N, ignore_index, n_valid, 0,
+                     static_cast<float*>(nullptr));
   TS_TRY(ts_host::check_launch("flce_count"));
   hipLaunchKernelGGL(flce_dscale, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, st, labels, N,
                      ignore_index, dloss, dloss_stride, n_valid, reduction == 0 ? 1 : 0, dscale);
@@ -1644,14 +1649,15 @@ extern "C" ts_status ts_flce_vocab_bwd(const void* hidden, int64_t ldh, const vo
   float* scale = reinterpret_cast<float*>(ws + lay.off_misc + 16);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
-  hipLaunchKernelGGL(flce_count, dim3(1), dim3(256), 0, st, labels, N, ignore_index, n_valid);
+  hipLaunchKernelGGL(flce_count, dim3(1), dim3(kOneWg), 0, st, labels, N, ignore_index, n_valid,
+                     reduction == 0 ? 1 : 0, scale);
   TS_TRY(ts_host::check_launch("flce_count"));
   hipLaunchKernelGGL(flce_vocab_merge, dim3((unsigned)((N + 63) / 64)), dim3(64), 0, st,
                      reinterpret_cast<const ShardStats*>(stats_all), P, N, labels, ignore_index,
                      lse_ws, rows_ws);
   TS_TRY(ts_host::check_launch("flce_vocab_merge"));
-  hipLaunchKernelGGL(flce_loss, dim3(1), dim3(256), 0, st, rows_ws, N, n_valid,
-                     reduction == 0 ? 1 : 0, loss, scale);
+  hipLaunchKernelGGL(flce_loss, dim3(1), dim3(kOneWg), 0, st, rows_ws, N, n_valid,
+                     reduction == 0 ? 1 : 0, loss);
   TS_TRY(ts_host::check_launch("flce_loss"));
   if (grad_hidden_partial == nullptr && grad_weight_shard == nullptr) return TS_OK;
   const int64_t ldl = logits_ld(Vp);
