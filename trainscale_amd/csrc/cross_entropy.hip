@@ -205,8 +205,7 @@ __global__ __launch_bounds__(kThreads) void ce_bwd_vec(
   GradRow r;
   r.dl = dloss[row * dloss_stride] * dloss_scale;
   r.lse2 = lse[row] * kLog2e;
-  r.keep = 1.f - smoothing;
-  r.av = smoothing / (float)V;
+  set_smoothing(r, smoothing, V);
   u32x4 buf[kBwdKv];
 #pragma unroll
   for (int k = 0; k < kBwdKv; ++k) {
@@ -281,7 +280,7 @@ __global__ __launch_bounds__(kRedThreads) void ce_loss_weight(
   if (used != nullptr) *used = h;
 }
 
-// The sum in double: its order then costs nothing in fp32.
+// The sum in double, rounded once after the division: its order then costs nothing in fp32.
 __global__ __launch_bounds__(kRedThreads) void ce_reduce_loss(
     const float* __restrict__ rows, const int64_t* __restrict__ labels, int64_t N,
     int64_t ignore_index, int mean, float div, float* __restrict__ out) {
@@ -305,7 +304,7 @@ __global__ __launch_bounds__(kRedThreads) void ce_reduce_loss(
   if (threadIdx.x != 0) return;
   double t = 0.0;
   for (int i = 0; i < kRedWaves; ++i) t += sums[i];
-  *out = (float)t / (mean ? (float)(c > 0 ? c : 1) : div);
+  *out = (float)(t / (mean ? (double)(c > 0 ? c : 1) : (double)div));
 }
 
 template <typename T>

@@ -106,9 +106,17 @@ __device__ inline void xform_vec(float (&z)[VE], const Xform& f) {
 struct GradRow {
   float dl;    // upstream gradient of this row
   float lse2;  // lse * log2(e)
-  float keep;  // 1 - a, what the label's element subtracts
-  float av;    // a / V
+  float keep;  // 1 - a in fp32, what the label's element subtracts
+  float av;    // a / V, what every other element subtracts
+  float avl;   // a / V and what keep lacks of 1 - a, what the label's subtracts before keep
 };
+// The label's element is most of a smoothed row's gradient norm, so it takes the small terms
+// first (one rounding near 1 - a, not two) and 1 - a in two floats.
+__device__ inline void set_smoothing(GradRow& r, float a, int64_t V) {
+  r.keep = 1.f - a;
+  r.av = a / (float)V;
+  r.avl = r.av + ((1.f - r.keep) - a);
+}
 
 // Gradient of one logit x.
 template <int kMode>
@@ -124,8 +132,8 @@ __device__ inline float grad1(float x, bool is_label, const GradRow& r, const Xf
     }
   }
   float g = fast_exp2(__builtin_fmaf(z, kLog2e, -r.lse2));
+  if constexpr (kMode != kPlain) g -= is_label ? r.avl : r.av;
   if (is_label) g -= r.keep;
-  if constexpr (kMode != kPlain) g -= r.av;
   if constexpr (kMode == kGeneral) g *= dz;
   return r.dl * g;
 }
@@ -158,8 +166,8 @@ __device__ inline void grad_vec(const float (&x)[VE], float (&g)[VE], int64_t la
 #pragma unroll
   for (int i = 0; i < VE; ++i) {
     float p = fast_exp2(__builtin_fmaf(z[i], kLog2e, -r.lse2));
+    if constexpr (kMode != kPlain) p -= i == lab ? r.avl : r.av;
     p = i == lab ? p - r.keep : p;
-    if constexpr (kMode != kPlain) p -= r.av;
     if constexpr (kMode == kGeneral) p *= dz[i];
     g[i] = r.dl * p;
   }
@@ -182,7 +190,9 @@ __device__ inline void fold1(float z, float& m, float& s) {
   }
 }
 
-// Loss of a row from its lse and (with smoothing) its sum of z; thread 0 only.
+// Loss of a row from its lse and (with smoothing) its sum of z; thread 0 only. The mix is
+// formed in double: the fp32 rounding of 1 - a is the same in every row, so a mean over rows
+// would keep it.
 template <int kMode, typename T>
 __device__ inline float row_loss(const T* xr, int64_t label, int64_t V, int64_t ignore_index,
                                  float l, float sz, float smoothing, const Xform& xf) {
@@ -190,7 +200,8 @@ __device__ inline float row_loss(const T* xr, int64_t label, int64_t V, int64_t 
   if (col < 0) return __builtin_nanf("");
   float out = l - xform1<kMode>(Elt<T>::load1(xr + col), xf);
   if (kMode != kPlain && smoothing != 0.f)
-    out = (1.f - smoothing) * out + smoothing * (l - sz / (float)V);
+    out = (float)((1.0 - (double)smoothing) * (double)out +
+                  (double)smoothing * (double)(l - sz / (float)V));
   return out;
 }
 
@@ -416,8 +427,7 @@ void ce_fused_vec(
       float, __builtin_amdgcn_readfirstlane(
                  __builtin_bit_cast(int, dloss[row * dloss_stride] * dloss_scale)));
   r.lse2 = l * kLog2e;
-  r.keep = 1.f - smoothing;
-  r.av = smoothing / (float)V;
+  set_smoothing(r, smoothing, V);
   if (has_tail && ec >= 0) Elt<G>::store1(gr + ec, grad1<kMode>(Elt<T>::load1(&xe), ec == label, r, xf));
   // The position of the label is uniform over the workgroup: its correction is a
   // uniform branch, and only the lane holding the label runs it.

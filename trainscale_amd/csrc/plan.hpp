@@ -413,8 +413,9 @@ TS_HOST_DEVICE inline int64_t tail_col(int64_t V, int t, int VE) {
 // per thread, rows of up to 256 a single wave (no barrier between waves to wait for).
 // Measured on MI355X (bf16, loss and gradient) against 1024 threads x 16 for every row:
 // [16384, 1000] 549 -> 17 us, [16384, 8192] 597 -> 87, [12500, 32000] 492 -> 279,
-// [6103, 65536] 312 -> 273; [16384, 128256] is the same kernel as before. fp32 gradients of 16-bit logits (`wide_grad`), which no
-// training path asks for, keep the one shape that holds every row.
+// [6103, 65536] 312 -> 273; [16384, 128256] is the same kernel as before. fp32 gradients of
+// 16-bit logits (`wide_grad`), which no training path asks for, keep the one shape that holds
+// every row.
 struct CeFusedPlan {
   int threads, kv;
 };
