@@ -1,0 +1,51 @@
+"""Cross-entropy rows whose first vectors lie far from the rest of the row, in both schedules
+and at every workgroup shape, against float64. A lane of the one-pass kernel sums its terms
+against its first vector's maximum: lanes with low references must not overflow together, nor
+may a lane whose reference lies far below the others' lose a large value."""
+import pytest
+import torch
+
+from test_gpu_ce_ragged import check, rows_at
+from trainscale_amd import ops
+
+pytestmark = pytest.mark.gpu
+BF, F32 = torch.bfloat16, torch.float32
+SHAPES = [(BF, 1000), (BF, 1003), (BF, 4000), (BF, 8192), (BF, 20001), (BF, 50257),
+          (BF, 131072), (torch.float16, 4099), (F32, 1000), (F32, 16389), (F32, 65536)]
+
+
+def both(x, V, labels, dl, a=0.0):
+    """(loss, lse, grad) of the one-pass and of the two-pass schedule."""
+    yield ops.ce_forward_backward(x, V, labels, dl, 1.0, -100, 0.0, 0.0, a)
+    loss, lse = ops.ce_forward(x, V, labels, -100, 0.0, 0.0, a)
+    grad = torch.empty_like(x)
+    ops.ce_backward(x, V, labels, lse, dl, grad, V, 1.0, -100, 0.0, 0.0, a)
+    yield loss, lse, grad
+
+
+@pytest.mark.parametrize("dtype,V", SHAPES)
+@pytest.mark.parametrize("a", [0.0, 0.1])
+def test_low_and_high_first_vectors(gpu, dtype, V, a):
+    ve = 4 if dtype == F32 else 8
+    leads = [t * ve for t in (64, 256, 512, 1024) if t * ve < V]  # first vectors, by workgroup
+    rows = []
+    for lead in leads:
+        for low, high in ((-84.0, 0.0), (0.0, 84.0), (-40.0, 0.0), (float("-inf"), 0.0)):
+            r = torch.full((V,), high)
+            r[:lead] = low
+            rows.append(r)
+        r = torch.full((V,), -20.0)  # lane 0's reference far below, its second vector the maximum
+        r[:ve], r[ve:2 * ve], r[lead] = -88.0, 0.0, 0.5
+        rows.append(r)
+    N = len(rows)
+    for off in (0, 1):
+        buf, x, labels = rows_at(N, V, V, off, dtype, gpu, V)
+        x.copy_(torch.stack(rows))
+        labels.fill_(V - 1)  # a finite logit in every row
+        dl = torch.linspace(0.5, 0.9, N, device=gpu)
+        if a:  # the smoothed loss of a row with -inf is inf
+            x.clamp_(min=-1e4)
+        for loss, lse, grad in both(x, V, labels, dl, a):
+            check(grad, loss, x, labels, dl, a=a)
+            torch.testing.assert_close(lse.double(), x.double().logsumexp(1), rtol=2.0 ** -22,
+                                       atol=2.0 ** -18)

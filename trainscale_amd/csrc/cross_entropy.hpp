@@ -261,6 +261,9 @@ constexpr uint32_t sign_bits() {
 // six at 8 and eight at 4.
 constexpr int fused_waves(int kv) { return kv >= 16 ? 4 : kv >= 8 ? 6 : 8; }
 
+// Largest sum of exp(z - m) that a lane's reference m serves for (see ce_fused_vec).
+constexpr float kLaneSumMax = 0x1p60f;
+
 template <typename T, typename G, int kMode, int kThr, int kKv, bool kAligned>
 __global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(fused_waves(kKv))))
 void ce_fused_vec(
@@ -346,12 +349,15 @@ void ce_fused_vec(
   // Each lane sums exp(z - m) over its vectors against one reference m, the
   // largest value of its first vector (0 if that vector is all -inf): per
   // element one unpack, one FMA, one exp and one add, with no running max or
-  // rescale. The sum is exact (terms that underflow lie below the resolution
-  // of a sum that holds exp(0) = 1) unless it ends outside [0.5, inf): a
-  // value more than 88 above m overflowed it, a NaN reached it, or an all
-  // -inf first vector left a sum of values far below 0. Such a lane (only
-  // with extreme logits) folds its vectors again from the registers with an
-  // exact online max and rescale. Lanes without vectors keep m = -inf, s = 0.
+  // rescale. Such a sum serves while it lies in [0.5, kLaneSumMax]: at 0.5 and
+  // more, terms that underflowed lie below its resolution; at 2^60 and less, the
+  // 1024 lanes' sums together stay finite, and a lane that the fold over the
+  // lanes rescales to zero (its m more than 87 below another lane's, whose sum
+  // is at least 0.5) held less than 2^60 2^-126, a 2^-65th of the row's sum.
+  // A lane outside that range (values more than 41 above m, a NaN, an all -inf
+  // first vector that left a sum of values far below 0) folds its vectors again
+  // from the registers with an exact online max and rescale: s in [1, VE * kKv]
+  // against the largest value. Lanes without vectors keep m = -inf, s = 0.
   float m = -INFINITY, mb = 0.f, s = 0.f, sz = 0.f;
   auto sum_exp = [&](const float (&z)[VE], float bias) {
     float cs = fast_exp2(__builtin_fmaf(z[0], kLog2e, -bias));
@@ -390,7 +396,7 @@ void ce_fused_vec(
     if ((k + 1) * kThr <= nvec) fold(buf[k], k == 0);
     else if ((int)threadIdx.x + k * kThr < nvec) fold(buf[k], k == 0);
   }
-  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s < INFINITY)) {
+  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s <= kLaneSumMax)) {
     m = -INFINITY;
     s = 0.f;
 #pragma unroll
