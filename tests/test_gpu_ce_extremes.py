@@ -49,3 +49,28 @@ def test_low_and_high_first_vectors(gpu, dtype, V, a):
             check(grad, loss, x, labels, dl, a=a)
             torch.testing.assert_close(lse.double(), x.double().logsumexp(1), rtol=2.0 ** -22,
                                        atol=2.0 ** -18)
+
+
+@pytest.mark.parametrize("dtype,V", SHAPES)
+@pytest.mark.parametrize("cap", [0.0, 20.0])
+def test_whole_vectors_of_nan(gpu, dtype, V, cap):
+    """A row holding one vector of NaN only, or of NaN and -inf, in a lane's first vector or a
+    later one, comes out NaN in both schedules; other rows do not."""
+    ve = 4 if dtype == F32 else 8
+    nvec = V // ve
+    at = [0, 63, 64 % nvec, 255 % nvec, 300 % nvec, nvec - 1]
+    N = 2 * len(at) + 1
+    for off in (0, 1):
+        buf, x, labels = rows_at(N, V, V, off, dtype, gpu, V)
+        labels.fill_(V - 1)
+        for i, v in enumerate(at):
+            for r in (2 * i, 2 * i + 1):
+                x[r, v * ve:(v + 1) * ve] = float("nan")
+            if cap == 0.0:
+                x[2 * i + 1, v * ve:v * ve + ve - 1] = float("-inf")
+        dl = torch.ones(N, device=gpu)
+        loss, lse, grad = ops.ce_forward_backward(x, V, labels, dl, 1.0, -100, 0.0, cap)
+        loss2, lse2 = ops.ce_forward(x, V, labels, -100, 0.0, cap)
+        for t in (loss, lse, loss2, lse2):
+            assert bool(t[:-1].isnan().all()) and bool(t[-1:].isfinite().all())
+        assert bool(grad[:-1].isnan().all()) and bool(grad[-1:].isfinite().all())

@@ -404,11 +404,12 @@ void ce_fused_vec(
       if ((int)threadIdx.x + k * kThr < nvec) {
         float z[VE];
         values(buf[k], z);
+        // mn is -inf only while every value is -inf, whose terms are 0, or NaN, which
+        // __builtin_fmaxf drops: its term makes s NaN, and s stays so
         const float mn = __builtin_fmaxf(m, vmax(z));
-        if (mn != -INFINITY) {
-          s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) + sum_exp(z, mn * kLog2e);
-          m = mn;
-        }
+        s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) +
+            sum_exp(z, mn == -INFINITY ? 0.f : mn * kLog2e);
+        m = mn;
       }
     }
   }
