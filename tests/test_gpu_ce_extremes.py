@@ -74,3 +74,35 @@ def test_whole_vectors_of_nan(gpu, dtype, V, cap):
         for t in (loss, lse, loss2, lse2):
             assert bool(t[:-1].isnan().all()) and bool(t[-1:].isfinite().all())
         assert bool(grad[:-1].isnan().all()) and bool(grad[-1:].isfinite().all())
+
+
+@pytest.mark.parametrize("dtype,V", SHAPES)
+@pytest.mark.parametrize("low", ["lowest", -1e38, -1e9, 3e38])
+def test_masked_with_the_lowest_value(gpu, dtype, V, low):
+    """Logits at their type's lowest value, as masks leave them: in the first vectors, in one
+    lane's, in all columns but one, in all columns; and logits near the largest."""
+    low = torch.finfo(dtype).min if low == "lowest" else low
+    if dtype == torch.float16 and abs(low) > 65504:
+        pytest.skip("beyond fp16")
+    ve = 4 if dtype == F32 else 8
+    leads = [t * ve for t in (1, 64, 256, 512, 1024) if t * ve < V]
+    N = len(leads) + 3
+    for off in (0, 1):
+        buf, x, labels = rows_at(N, V, V, off, dtype, gpu, V)
+        labels.fill_(V - 1)
+        for r, lead in enumerate(leads):
+            x[r, :lead] = low
+        x[N - 3, :V - 1] = low  # one column left
+        x[N - 2, V // 2:V - 1] = low
+        x[N - 1] = low  # nothing left: every logit is the maximum
+        dl = torch.ones(N, device=gpu)
+        if low > 0:  # the gradient needs lse * log2 e, which is past fp32 here
+            lse = ops.ce_forward_backward(x, V, labels, dl)[1]
+            for l in (lse, ops.ce_forward(x, V, labels)[1]):
+                torch.testing.assert_close(l.double(), x.double().logsumexp(1), rtol=2.0 ** -23,
+                                           atol=0)
+            continue
+        for loss, lse, grad in both(x, V, labels, dl):
+            assert lse[N - 1] == x[N - 1, 0].float() + torch.tensor(float(V)).log()
+            assert bool(loss[N - 1].isfinite())
+            check(grad[:N - 1], loss[:N - 1], x[:N - 1], labels[:N - 1], dl[:N - 1])

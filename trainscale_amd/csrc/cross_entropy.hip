@@ -117,12 +117,16 @@ __global__ __launch_bounds__(kThreads) void ce_fwd_vec(const T* __restrict__ log
       s = s == 0.f ? 0.f : s * fast_exp2((m - lm) * kLog2e);
       m = lm;
     }
-    // m is -inf only while every value seen is -inf: their terms are 0.
-    const float mb = m == -INFINITY ? 0.f : m * kLog2e;
+    if (fabsf(m) < kRefMax) {
+      const float mb = m * kLog2e;
 #pragma unroll
-    for (int u = 0; u < kUnroll; ++u)
+      for (int u = 0; u < kUnroll; ++u)
 #pragma unroll
-      for (int i = 0; i < VE; ++i) s += fast_exp2(__builtin_fmaf(z[u][i], kLog2e, -mb));
+        for (int i = 0; i < VE; ++i) s += fast_exp2(__builtin_fmaf(z[u][i], kLog2e, -mb));
+    } else {
+#pragma unroll
+      for (int u = 0; u < kUnroll; ++u) s += sum_exp_far<VE>(z[u], m);
+    }
   }
   // Tail: fewer than kThreads*kUnroll vectors remain.
   for (int64_t v = ts_plan::chunk_vec(c, 0, threadIdx.x, kThreads, kUnroll); v < nvec;
@@ -140,10 +144,13 @@ __global__ __launch_bounds__(kThreads) void ce_fwd_vec(const T* __restrict__ log
       s = s == 0.f ? 0.f : s * fast_exp2((m - lm) * kLog2e);
       m = lm;
     }
-    // m is -inf only while every value seen is -inf: their terms are 0.
-    const float mb = m == -INFINITY ? 0.f : m * kLog2e;
+    if (fabsf(m) < kRefMax) {
+      const float mb = m * kLog2e;
 #pragma unroll
-    for (int i = 0; i < VE; ++i) s += fast_exp2(__builtin_fmaf(z[i], kLog2e, -mb));
+      for (int i = 0; i < VE; ++i) s += fast_exp2(__builtin_fmaf(z[i], kLog2e, -mb));
+    } else {
+      s += sum_exp_far<VE>(z, m);
+    }
   }
   if (ec >= 0) {
     const float ze = xform1<kMode>(Elt<T>::load1(xr + ec), xf);

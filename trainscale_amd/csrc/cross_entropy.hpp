@@ -179,6 +179,23 @@ __device__ inline int64_t tail_col(int64_t V) {
   return ts_plan::tail_col(V, (int)threadIdx.x, VE);
 }
 
+// exp(z - m) formed as exp2(fma(z, log2 e, -m log2 e)) carries the rounding of m log2 e, up to
+// 2^-24 |m| log2 e in the exponent: below this magnitude at most 0.07, past it as much as the
+// sum's whole range, and the product overflows where logits are masked with their type's
+// lowest value (-3.4e38 in bf16 and fp32). References at or past it take sum_exp_far.
+constexpr float kRefMax = 0x1p20f;
+
+// Sum of exp(z - m) over a vector for any reference m that is no less than its values. m is
+// -inf only while every value seen is -inf, whose terms are 0, or NaN.
+template <int VE>
+__device__ inline float sum_exp_far(const float (&z)[VE], float m) {
+  const float ref = m == -INFINITY ? 0.f : m;
+  float cs = fast_exp2((z[0] - ref) * kLog2e);
+#pragma unroll
+  for (int i = 1; i < VE; ++i) cs += fast_exp2((z[i] - ref) * kLog2e);
+  return cs;
+}
+
 // Adds the value z to an online (max, sum of exp) pair; nothing for -inf.
 __device__ inline void fold1(float z, float& m, float& s) {
   const float mn = __builtin_fmaxf(m, z);
@@ -354,8 +371,8 @@ void ce_fused_vec(
   // 1024 lanes' sums together stay finite, and a lane that the fold over the
   // lanes rescales to zero (its m more than 87 below another lane's, whose sum
   // is at least 0.5) held less than 2^60 2^-126, a 2^-65th of the row's sum.
-  // A lane outside that range (values more than 41 above m, a NaN, an all -inf
-  // first vector that left a sum of values far below 0) folds its vectors again
+  // A lane outside that range (values more than 41 above m, a NaN, a reference
+  // past kRefMax, an all -inf first vector that left a sum of values far below 0) folds its vectors again
   // from the registers with an exact online max and rescale: s in [1, VE * kKv]
   // against the largest value. Lanes without vectors keep m = -inf, s = 0.
   float m = -INFINITY, mb = 0.f, s = 0.f, sz = 0.f;
@@ -396,7 +413,7 @@ void ce_fused_vec(
     if ((k + 1) * kThr <= nvec) fold(buf[k], k == 0);
     else if ((int)threadIdx.x + k * kThr < nvec) fold(buf[k], k == 0);
   }
-  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s <= kLaneSumMax)) {
+  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s <= kLaneSumMax && fabsf(m) < kRefMax)) {
     m = -INFINITY;
     s = 0.f;
 #pragma unroll
@@ -404,11 +421,9 @@ void ce_fused_vec(
       if ((int)threadIdx.x + k * kThr < nvec) {
         float z[VE];
         values(buf[k], z);
-        // mn is -inf only while every value is -inf, whose terms are 0, or NaN, which
-        // __builtin_fmaxf drops: its term makes s NaN, and s stays so
+        // __builtin_fmaxf drops NaN, whose term makes s NaN, and s stays so
         const float mn = __builtin_fmaxf(m, vmax(z));
-        s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) +
-            sum_exp(z, mn == -INFINITY ? 0.f : mn * kLog2e);
+        s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) + sum_exp_far<VE>(z, mn);
         m = mn;
       }
     }
