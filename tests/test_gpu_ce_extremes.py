@@ -106,3 +106,24 @@ def test_masked_with_the_lowest_value(gpu, dtype, V, low):
             assert lse[N - 1] == x[N - 1, 0].float() + torch.tensor(float(V)).log()
             assert bool(loss[N - 1].isfinite())
             check(grad[:N - 1], loss[:N - 1], x[:N - 1], labels[:N - 1], dl[:N - 1])
+
+
+@pytest.mark.parametrize("V", [1001, 4003, 16389, 65536])
+@pytest.mark.parametrize("low", [0.0, -10.0, -20.0, -30.0, -40.0])
+def test_lse_does_not_depend_on_the_reference(gpu, V, low):
+    """lse to about an ulp wherever the lanes' first vectors lie. Its rms error in ulps: the last
+    rounding (0.29); logf, at most 1 (0.3); v_exp_f32's ulp, alike in many terms (1.2e-7 of the
+    sum, 0.25 of an lse between 4 and 8); the roundings of the sum (2^-24 of it, 0.13) and of
+    exponents of up to 60 (8e-7 a term, averaged over hundreds of them): together below 0.9."""
+    for lead in (256, 1024, 2048, 4096):
+        if lead > V // 2:
+            break
+        g = torch.Generator(device=gpu).manual_seed(V + lead)
+        x = torch.randn(512, V, generator=g, device=gpu)
+        x[:, :lead] += low
+        labels = torch.zeros(512, dtype=torch.long, device=gpu)
+        lse = ops.ce_forward_backward(x, V, labels, torch.ones(1, device=gpu))[1]
+        ref = x.double().logsumexp(1)
+        ulp = 2.0 ** (ref.log2().floor() - 23)
+        err = (lse.double() - ref) / ulp
+        assert err.pow(2).mean().sqrt().item() <= 0.9, (lead, err.pow(2).mean().sqrt().item())

@@ -240,6 +240,25 @@ __device__ inline float row_loss(const T* xr, int64_t label, int64_t V, int64_t 
 // corrected by the one lane that holds it.
 // ---------------------------------------------------------------------------
 
+// Moves a lane's (m, sum of exp2(z log2 e - mb)) pair, mb = m log2 e rounded, to a reference
+// next to its sum: s about in [0.5, 1) and m + log(s) the lane's log-sum, without the roundings
+// of mb and of log2 e (r is what mb lacks of m log2 e) and, where m lay far below the lane's
+// values, without two large terms that cancel. What the new m lost in its rounding goes into s.
+// Rms error of lse at [512, 1001] fp32 N(0, 1), the first 256 columns 20 lower: 1.46 ulp
+// without, 0.62 now, as for rows that do not begin so; 0.64 -> 0.56 ulp for those.
+__device__ inline void settle(float& m, float mb, float& s) {
+  constexpr float kLog2eLo = (float)(1.4426950408889634 - (double)kLog2e);
+  constexpr float kLn2Lo = (float)(0.6931471805599453 - (double)kLn2);
+  const float r = __builtin_fmaf(m, kLog2eLo, __builtin_fmaf(m, kLog2e, -mb));
+  const float k = (float)__builtin_amdgcn_frexp_expf(s);
+  const float m1 = __builtin_fmaf(k, kLn2, m);
+  const float lost =
+      __builtin_fmaf(k, kLn2, m - m1) + __builtin_fmaf(k, kLn2Lo, -r * kLn2);
+  const float s1 = __builtin_amdgcn_frexp_mantf(s);
+  s = __builtin_fmaf(s1, lost, s1);
+  m = m1;
+}
+
 // Row lse (and, with smoothing, the row sum of z) from every thread's online
 // (max, sum of exp) pair. lds holds 3 * kNW floats. One barrier: the
 // caller must not write lds again without another barrier in between.
@@ -278,8 +297,16 @@ constexpr uint32_t sign_bits() {
 // six at 8 and eight at 4.
 constexpr int fused_waves(int kv) { return kv >= 16 ? 4 : kv >= 8 ? 6 : 8; }
 
-// Largest sum of exp(z - m) that a lane's reference m serves for (see ce_fused_vec).
-constexpr float kLaneSumMax = 0x1p60f;
+// Largest sum of exp(z - m) that a lane's reference m serves for (see ce_fused_vec). The lower
+// the bound, the nearer the exponents of the terms that matter are to 0, where they are rounded
+// finest; but lanes that hold a logit above it, log(bound) higher than their first vector, pay a
+// second fold, and a workgroup waits for its slowest wave. With 2^20, lse errors do not depend
+// on where the first vectors lie; with 2^60 they grow from 0.6 to 0.9 ulp rms where these lie 30
+// below the row. Measured on MI355X with 8 logits a row 22 high among N(0, 2), bf16, 2^16
+// against 2^60: [8192, 32000] 185 and 181 us, [8191, 50257] 373 and 369, but [8192, 128256], a
+// lone 1024-thread workgroup a CU, 776 and 729: aligned rows of that shape keep 2^60.
+template <int kThr, bool kAligned>
+constexpr float lane_sum_max() { return kThr == 1024 && kAligned ? 0x1p60f : 0x1p20f; }
 
 template <typename T, typename G, int kMode, int kThr, int kKv, bool kAligned>
 __global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(fused_waves(kKv))))
@@ -290,6 +317,7 @@ void ce_fused_vec(
     G* __restrict__ grad, int64_t ld_grad) {
   constexpr int VE = Elt<T>::kVec;
   constexpr int kNW = kThr / kWave;
+  constexpr float kLaneSumMax = lane_sum_max<kThr, kAligned>();
   constexpr int kGradBytes = VE * (int)sizeof(G);  // grad bytes per logits vector
   __shared__ float lds[3 * kNW];
   const int64_t row = blockIdx.x;
@@ -366,13 +394,11 @@ void ce_fused_vec(
   // Each lane sums exp(z - m) over its vectors against one reference m, the
   // largest value of its first vector (0 if that vector is all -inf): per
   // element one unpack, one FMA, one exp and one add, with no running max or
-  // rescale. Such a sum serves while it lies in [0.5, kLaneSumMax]: at 0.5 and
-  // more, terms that underflowed lie below its resolution; at 2^60 and less, the
-  // 1024 lanes' sums together stay finite, and a lane that the fold over the
-  // lanes rescales to zero (its m more than 87 below another lane's, whose sum
-  // is at least 0.5) held less than 2^60 2^-126, a 2^-65th of the row's sum.
-  // A lane outside that range (values more than 41 above m, a NaN, a reference
-  // past kRefMax, an all -inf first vector that left a sum of values far below 0) folds its vectors again
+  // rescale. Such a sum serves while it lies in [0.5, lane_sum_max]: terms that
+  // underflowed are then below its resolution, and settle brings it next to its
+  // reference, so that no fold over the lanes overflows with it or loses it.
+  // Other lanes (values far above m, a NaN, a reference past kRefMax, an all -inf
+  // first vector that left a sum of values far below 0) fold their vectors again
   // from the registers with an exact online max and rescale: s in [1, VE * kKv]
   // against the largest value. Lanes without vectors keep m = -inf, s = 0.
   float m = -INFINITY, mb = 0.f, s = 0.f, sz = 0.f;
@@ -413,7 +439,9 @@ void ce_fused_vec(
     if ((k + 1) * kThr <= nvec) fold(buf[k], k == 0);
     else if ((int)threadIdx.x + k * kThr < nvec) fold(buf[k], k == 0);
   }
-  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s <= kLaneSumMax && fabsf(m) < kRefMax)) {
+  if (s >= 0.5f && s <= kLaneSumMax && fabsf(m) < kRefMax) {
+    settle(m, mb, s);
+  } else if ((int)threadIdx.x < nvec) {
     m = -INFINITY;
     s = 0.f;
 #pragma unroll
