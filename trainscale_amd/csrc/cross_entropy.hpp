@@ -299,14 +299,19 @@ constexpr int fused_waves(int kv) { return kv >= 16 ? 4 : kv >= 8 ? 6 : 8; }
 
 // Largest sum of exp(z - m) that a lane's reference m serves for (see ce_fused_vec). The lower
 // the bound, the nearer the exponents of the terms that matter are to 0, where they are rounded
-// finest; but lanes that hold a logit above it, log(bound) higher than their first vector, pay a
-// second fold, and a workgroup waits for its slowest wave. With 2^20, lse errors do not depend
-// on where the first vectors lie; with 2^60 they grow from 0.6 to 0.9 ulp rms where these lie 30
-// below the row. Measured on MI355X with 8 logits a row 22 high among N(0, 2), bf16, 2^16
-// against 2^60: [8192, 32000] 185 and 181 us, [8191, 50257] 373 and 369, but [8192, 128256], a
-// lone 1024-thread workgroup a CU, 776 and 729: aligned rows of that shape keep 2^60.
-template <int kThr, bool kAligned>
-constexpr float lane_sum_max() { return kThr == 1024 && kAligned ? 0x1p60f : 0x1p20f; }
+// finest; but a wave with a lane that holds a logit log(bound) above its first vector folds its
+// vectors twice. With 2^20 lse errors do not depend on where the first vectors lie; with 2^40
+// and 2^60 they grow from 0.6 to 0.7 and 0.9 ulp rms where these lie 20 and 30 below the row.
+// 2^20 is for the rows that older kernels folded with an exact online max (short ones and
+// those off 16-byte boundaries; measured on MI355X, [4096, 50257] bf16 of N(0, 4): 191 against
+// 189 us with 2^60). Aligned longer rows had no such fold: [8192, 128256] with 64 logits a row
+// 22 high takes 796 us with 2^16, 732 with 2^60. With transforms a second fold costs most
+// ([4096, 50257], softcap 30, N(0, 6): 297 us with 2^20, 253 with 2^40), and the rounding of the
+// transformed logits themselves covers the difference.
+template <int kMode, int kThr, int kKv, bool kAligned>
+constexpr float lane_sum_max() {
+  return kAligned && kThr * kKv > 1024 ? 0x1p60f : kMode == kGeneral ? 0x1p40f : 0x1p20f;
+}
 
 template <typename T, typename G, int kMode, int kThr, int kKv, bool kAligned>
 __global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(fused_waves(kKv))))
@@ -317,7 +322,7 @@ void ce_fused_vec(
     G* __restrict__ grad, int64_t ld_grad) {
   constexpr int VE = Elt<T>::kVec;
   constexpr int kNW = kThr / kWave;
-  constexpr float kLaneSumMax = lane_sum_max<kThr, kAligned>();
+  constexpr float kLaneSumMax = lane_sum_max<kMode, kThr, kKv, kAligned>();
   constexpr int kGradBytes = VE * (int)sizeof(G);  // grad bytes per logits vector
   __shared__ float lds[3 * kNW];
   const int64_t row = blockIdx.x;
