@@ -4,6 +4,7 @@
 // instantiations (row shapes, modes, alignment), so each data type compiles in its own file.
 #pragma once
 
+#include <float.h>
 #include <math.h>
 
 #include "common.hpp"
@@ -22,38 +23,59 @@ enum Mode : int { kPlain = 0, kSmooth = 1, kGeneral = 2 };
 struct Xform {
   float scale;    // 1 when off
   float softcap;  // 0 = off
-  float inv_cap;  // 1 / softcap
+  float inv_cap, inv_cap_lo;  // 1 / softcap in two floats, both above 0 (cap_quot)
 };
 inline Xform make_xform(float logit_scale, float softcap) {
-  return Xform{logit_scale != 0.f ? logit_scale : 1.f, softcap,
-               softcap != 0.f ? 1.f / softcap : 0.f};
+  Xform f{logit_scale != 0.f ? logit_scale : 1.f, softcap, 0.f, 0.f};
+  if (softcap == 0.f) return f;
+  const double inv = 1.0 / (double)softcap;
+  if (inv > (double)FLT_MAX) {  // softcap below 2^-128
+    f.inv_cap = FLT_MAX;
+  } else {
+    f.inv_cap = (float)inv;
+    if ((double)f.inv_cap >= inv) f.inv_cap = nextafterf(f.inv_cap, 0.f);
+    f.inv_cap_lo = (float)(inv - (double)f.inv_cap);
+  }
+  if (f.inv_cap_lo == 0.f) f.inv_cap_lo = FLT_TRUE_MIN;
+  return f;
+}
+// z / softcap, rounded once. z times the rounded reciprocal alone carries that one's error in
+// every element (at softcap 30 a relative 5.2e-8); the low part is above 0 so that infinite z
+// meet no product of infinity and 0 or of two signs.
+__device__ inline float cap_quot(float z, const Xform& f) {
+  return __builtin_fmaf(z, f.inv_cap, z * f.inv_cap_lo);
 }
 inline Mode mode_of(float logit_scale, float softcap, float smoothing) {
   return logit_scale != 0.f || softcap != 0.f ? kGeneral : smoothing != 0.f ? kSmooth : kPlain;
 }
 
-// tanh to about one fp32 ulp in two ranges. Below kTanhSmall: x + x^3 P(x^2), P of degree 5
-// fitted for least relative error over [0, 0.75] (1.7e-9 before rounding, 0.75 ulp in fp32
-// arithmetic). From there on: 1 - 2 / (1 + exp(2|x|)) with v_exp_f32 and v_rcp_f32 (each
-// within 1 ulp), whose error the subtraction of a term below 0.37 keeps under 2 ulps. A
-// vector whose values are all small in every lane of the wave skips the second form, which
-// costs twice the first. The device library's tanhf made the softcapped kernels
-// VALU-bound: at [4096, 32000] bf16, softcap 30, the forward took 99 us and now takes 61,
-// the backward 132 and 95.
-constexpr float kTanhSmall = 0.75f;
+// tanh in two ranges, as accurate as the device library's tanhf. Below kTanhSmall:
+// x + x^3 P(x^2), P of degree 5 fitted over [0, 0.85] for least relative error, four times
+// closer near 0 (2.7e-9 there, 1.3e-8 at the end, before rounding). From there on:
+// 1 - 2 / (1 + exp(2|x|)) with v_exp_f32 and v_rcp_f32 (each within 1 ulp), the exponent
+// shifted by kShift, which keeps its rounding small where 2 / (1 + e) still counts;
+// kPower = 2^kShift (1 + 3e-8), whose excess makes up for the rounding of 2 log2 e. A vector
+// whose values are all small in every lane of the wave skips the second form, which costs
+// twice the first. tanhf made the softcapped kernels VALU-bound: at [4096, 32000] bf16,
+// softcap 30, the forward took 98 us and now takes 62, the backward 129 and 98. Rms error of the
+// softcapped logit in ulps, tanhf(x / c) against these and cap_quot, c = 30: 0.530 and 0.517 for
+// |x / c| below 0.75, 0.464 and 0.460 from there to 1.5, 0.399 and 0.400 from there to 4.
+constexpr float kTanhSmall = 0.85f;
 __device__ inline float tanh_small(float x) {
   const float s = x * x;
-  float p = 0.00173693569f;
-  p = __builtin_fmaf(p, s, -0.00765725551f);
-  p = __builtin_fmaf(p, s, 0.0214520339f);
-  p = __builtin_fmaf(p, s, -0.0538927242f);
-  p = __builtin_fmaf(p, s, 0.133326948f);
-  p = __builtin_fmaf(p, s, -0.333333164f);
+  float p = 0.001508764f;
+  p = __builtin_fmaf(p, s, -0.007290129f);
+  p = __builtin_fmaf(p, s, 0.021238737f);
+  p = __builtin_fmaf(p, s, -0.053839035f);
+  p = __builtin_fmaf(p, s, 0.13332148f);
+  p = __builtin_fmaf(p, s, -0.333333f);
   return __builtin_fmaf(p, s * x, x);
 }
 __device__ inline float tanh_large(float x) {
-  const float e = fast_exp2(fabsf(x) * (2.f * kLog2e));
-  return copysignf(__builtin_fmaf(-2.f, __builtin_amdgcn_rcpf(1.f + e), 1.f), x);
+  constexpr float kShift = 2.974609375f, kPower = 7.8604364f;
+  const float e = fast_exp2(__builtin_fmaf(fabsf(x), 2.f * kLog2e, -kShift));
+  const float r = __builtin_amdgcn_rcpf(__builtin_fmaf(kPower, e, 1.f));
+  return copysignf(__builtin_fmaf(-2.f, r, 1.f), x);
 }
 // |x| < kTanhSmall is false for NaN, and tanh_large(NaN) is NaN.
 __device__ inline float tanh1(float x) {
@@ -71,8 +93,10 @@ __device__ inline void tanh_vec(const float (&u)[VE], float (&t)[VE]) {
   // fmaxf drops a NaN, whose tanh_small is NaN too
   if (__builtin_amdgcn_ballot_w64(um >= kTanhSmall) != 0) {
 #pragma unroll
-    for (int i = 0; i < VE; ++i)
-      if (!(fabsf(u[i]) < kTanhSmall)) t[i] = tanh_large(u[i]);
+    for (int i = 0; i < VE; ++i) {
+      const float l = tanh_large(u[i]);
+      t[i] = fabsf(u[i]) < kTanhSmall ? t[i] : l;
+    }
   }
 }
 
@@ -81,7 +105,7 @@ template <int kMode>
 __device__ inline float xform1(float x, const Xform& f) {
   if constexpr (kMode == kGeneral) {
     x *= f.scale;
-    if (f.softcap != 0.f) x = f.softcap * tanh1(x * f.inv_cap);
+    if (f.softcap != 0.f) x = f.softcap * tanh1(cap_quot(x, f));
   }
   return x;
 }
@@ -94,7 +118,7 @@ __device__ inline void xform_vec(float (&z)[VE], const Xform& f) {
     if (f.softcap != 0.f) {
       float u[VE], t[VE];
 #pragma unroll
-      for (int i = 0; i < VE; ++i) u[i] = z[i] * f.inv_cap;
+      for (int i = 0; i < VE; ++i) u[i] = cap_quot(z[i], f);
       tanh_vec<VE>(u, t);
 #pragma unroll
       for (int i = 0; i < VE; ++i) z[i] = f.softcap * t[i];
@@ -126,7 +150,7 @@ __device__ inline float grad1(float x, bool is_label, const GradRow& r, const Xf
     z *= f.scale;
     dz = f.scale;
     if (f.softcap != 0.f) {
-      const float t = tanh1(z * f.inv_cap);
+      const float t = tanh1(cap_quot(z, f));
       z = f.softcap * t;
       dz = (1.f - t * t) * f.scale;
     }
@@ -154,7 +178,7 @@ __device__ inline void grad_vec(const float (&x)[VE], float (&g)[VE], int64_t la
     if (f.softcap != 0.f) {
       float u[VE], t[VE];
 #pragma unroll
-      for (int i = 0; i < VE; ++i) u[i] = z[i] * f.inv_cap;
+      for (int i = 0; i < VE; ++i) u[i] = cap_quot(z[i], f);
       tanh_vec<VE>(u, t);
 #pragma unroll
       for (int i = 0; i < VE; ++i) {
@@ -441,7 +465,8 @@ void ce_fused_vec(
   for (int k = 0; k < kKv; ++k) {
     // Vectors every thread holds take a uniform branch; only the row's last
     // partial sweep tests each lane.
-    if ((k + 1) * kThr <= nvec) fold(buf[k], k == 0);
+    // With transforms one copy of their code serves both.
+    if (kMode != kGeneral && (k + 1) * kThr <= nvec) fold(buf[k], k == 0);
     else if ((int)threadIdx.x + k * kThr < nvec) fold(buf[k], k == 0);
   }
   if (s >= 0.5f && s <= kLaneSumMax && fabsf(m) < kRefMax) {
@@ -510,9 +535,12 @@ void ce_fused_vec(
     } else {
       grad_vec<kMode, VE>(z, g, -1, r, xf);
       if (k == klab && (int)threadIdx.x == tlab) {
+        float zl = z[0];
 #pragma unroll
-        for (int i = 0; i < VE; ++i)
-          if (i == elab) g[i] = grad1<kMode>(z[i], true, r, xf);
+        for (int i = 1; i < VE; ++i) zl = i == elab ? z[i] : zl;
+        const float gl = grad1<kMode>(zl, true, r, xf);
+#pragma unroll
+        for (int i = 0; i < VE; ++i) g[i] = i == elab ? gl : g[i];
       }
     }
     if constexpr (kGradBytes == 32) {
