@@ -164,7 +164,8 @@ def test_small_shapes(gpu, N, H, V):
     w = (0.05 * torch.randn(V, H, device=gpu)).to(BF)
     labels = torch.randint(0, V, (N,), device=gpu)
     labels[::20] = -100
-    check_against_oracle(h, w, labels)
+    for chunk in (None, 256):
+        check_against_oracle(h, w, labels, chunk=chunk)
 
 
 @pytest.mark.parametrize("chunk", [256, 512])
@@ -205,11 +206,12 @@ def test_exact_logits_pin_the_gemms(gpu):
     w = (torch.randint(-2, 3, (V, H), device=gpu).float() / 2).to(BF)
     labels = torch.randint(0, V, (N,), device=gpu)
     labels[5] = -100
-    loss, rows, lse, gh, gw = linear_ce_forward_backward(h, w, labels, reduction="sum")
+    loss, rows, lse, gh, gw = linear_ce_forward_backward(h, w, labels, reduction="sum",
+                                                         chunk_tokens=256)
     ref_loss, _, _, ref_rows, ref_lse = oracle.linear_ce(
         h, w, labels, reduction="sum", bf16_logits=True, return_rows=True)
     torch.testing.assert_close(rows.cpu(), ref_rows, rtol=2e-6, atol=2e-5)
-    ref = make_ref(h, w, labels, "sum", token_chunk=_token_chunk(N, V, None) or N)
+    ref = make_ref(h, w, labels, "sum", token_chunk=_token_chunk(N, V, 256))
     # exact logits: the kernel's dlogits can differ from the reference's only by the
     # rounding of values that the two exp implementations put on either side of a midpoint
     assert ref.d_changed <= ref.d_total // 1000, ref.d_changed
@@ -269,7 +271,7 @@ def test_vocab_and_hidden_not_multiples_of_8(gpu, N, H, V):
     """V not a multiple of 8 (GPT-2's 50257): the library pads its logits rows to whole
     16-byte vectors and masks the columns past V; H not a multiple of 8: the wrapper
     zero-pads hidden and weight. Every schedule against the oracle: the one-call schedule
-    (default token chunks with an fp32 and a bf16 grad_weight sum, one chunk), the
+    (the default chunk, and chunks of 256 with an fp32 and a bf16 grad_weight sum), the
     two-pass schedule (default and 256-column vocabulary chunks) and, through make_ref,
     the stored-logits schedule."""
     torch.manual_seed(N + H + V)
@@ -278,7 +280,7 @@ def test_vocab_and_hidden_not_multiples_of_8(gpu, N, H, V):
     labels = torch.randint(0, V, (N,), device=gpu)
     labels[::13] = -100
     labels[1] = V - 1  # the last column, in the partial last vector when V % 8 != 0
-    for chunk, accum in ((None, "fp32"), (None, "bf16"), (0, "bf16")):
+    for chunk, accum in ((None, "fp32"), (None, "bf16"), (256, "fp32"), (256, "bf16")):
         _, gh, gw = check_against_oracle(h, w, labels, chunk=chunk, accum=accum)
         assert gh.shape == (N, H) and gw.shape == (V, H)
     for chunk in (None, 256):
@@ -575,14 +577,14 @@ def test_one_call_schedule_odd_tokens(gpu):
     h = torch.randn(N, H, device=gpu).to(BF).requires_grad_()
     w = (0.05 * torch.randn(V, H, device=gpu)).to(BF).requires_grad_()
     labels = torch.randint(0, V, (N,), device=gpu)
-    loss = fused_linear_cross_entropy(h, w, labels, schedule="fused")
+    loss = fused_linear_cross_entropy(h, w, labels, schedule="fused", chunk_tokens=256)
     loss.backward()
     ref_loss, _, _ = oracle.linear_ce(h.detach(), w.detach(), labels, bf16_logits=True)
     assert abs(loss.item() - float(ref_loss)) <= 1e-5 * abs(float(ref_loss))
     assert h.grad.shape == (N, H)
     # the kernel runs N rounded up to 8 rows (the extra rows ignored) in chunks of 256 with
     # grad_weight summed in bf16 (the module's default)
-    tc = _token_chunk(N + 5, V, None)
+    tc = _token_chunk(N + 5, V, 256)
     assert tc == 256
     ref = make_ref(h.detach(), w.detach(), labels, token_chunk=tc)
     check_grads(h.grad, w.grad, ref, gw_mode="bf16_run", what="odd tokens")

@@ -10,7 +10,8 @@ from trainscale_amd.loss import linear_ce as L
 BF = torch.bfloat16
 
 
-@pytest.mark.parametrize("N,V,rows", [(1, 8, 0), (512, 4095, 256), (512, 4096, 0), (256, 1 << 22, 0), (4096, 1 << 17, 0),
+@pytest.mark.parametrize("N,V,rows", [(1, 8, 0), (512, 1000, 0), (1 << 16, 8, 0),
+                                      (256, 1 << 22, 0), (4096, 1 << 17, 0),
                                       (4097, 1 << 17, 2304), (8192, 128256, 4096),
                                       (4099, (1 << 17) - 5, 2304), (300, 1 << 21, 256)])
 def test_token_chunk(N, V, rows):

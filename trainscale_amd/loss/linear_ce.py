@@ -62,12 +62,11 @@ __all__ = ["LinearCrossEntropyFunction", "FusedLinearCrossEntropyFunction",
 # the scratch that half of C5's tokens take (N = 8192: 1.05 GB). Measured on MI355X,
 # two chunks against one: N = 512, H = 4096, V = 128256 2.27 -> 1.60 ms; 2048 tokens
 # 5.78 -> 5.19; 4096 tokens 10.6 -> 10.0; 2045, 768, 50257 726 -> 615 us; at C5, above
-# the bound, 20.08 and 19.77 ms (and 22.5 against 21.5 with four chunks and two). Vocabularies
-# smaller than any LM head's (below 4096 columns) keep the two chunks: nothing is gained there
-# but launches, and small inputs keep running the sum over chunks.
+# the bound, 20.08 and 19.77 ms (and 22.5 against 21.5 with four chunks and two); of
+# small vocabularies, 4096, 1024, 4000 243 -> 141 us, 512, 256, 1000 96 -> 51, 65536, 1024,
+# 4000 2439 and 2440.
 DEFAULT_TOKEN_CHUNKS = 2
 _ONE_CHUNK_BYTES = 1 << 30
-_ONE_CHUNK_MIN_V = 4096
 
 _REDUCTIONS = {"mean": 0, "sum": 1}
 TS_FLCE_GRADS, TS_FLCE_ACCUM_BF16 = 1, 2  # include/trainscale_amd.h
@@ -79,7 +78,7 @@ def _chunk_rows(N: int, V: int, chunk_tokens: Optional[int]) -> int:
     chunk while the bf16 logits take at most _ONE_CHUNK_BYTES, else half the tokens."""
     if chunk_tokens is not None:
         return int(chunk_tokens)
-    if V >= _ONE_CHUNK_MIN_V and N * _logits_ld(V) * 2 <= _ONE_CHUNK_BYTES:
+    if N * _logits_ld(V) * 2 <= _ONE_CHUNK_BYTES:
         return 0
     rows = -(-N // DEFAULT_TOKEN_CHUNKS)
     rows = -(-rows // 256) * 256
