@@ -22,27 +22,30 @@ int main() {
   for (long long nvec = 0; nvec <= 130; ++nvec) {
     const int f = rms_narrow_tpr(nvec);
     CHECK(f == 0 ? nvec == 0 || nvec > 32 : f >= nvec && (f == 8 || f == 16 || f == 32), "tpr");
-    for (long long rows : {1ll, 15ll, 16ll, 17ll, 127ll, 128ll, 129ll, 8192ll, 65537ll, 262144ll, 1ll << 30}) {
-      const RmsNarrowPlan p = rms_bwd_narrow_plan(rows, nvec);
-      if (nvec == 0 || nvec > 64) { CHECK(p.tpr == 0, "not narrow"); continue; }
-      CHECK(p.tpr >= nvec && p.tpr <= 64 && p.rpb * p.tpr == kNarrowBlock, "shape");
-      CHECK(p.grid >= 1 && p.grid <= kBwdGridTarget, "grid");
-      CHECK(p.grid * p.steps * p.rpb >= rows, "rows not covered");
-      CHECK((p.grid - 1) * p.steps * p.rpb < rows, "empty workgroup");
+    if (f != 0) CHECK(rms_fwd_plan(nvec).tpr == f && rms_fwd_plan(nvec).kv == 1, "forward lanes");
+    for (long long rows : {1ll, 15ll, 16ll, 17ll, 127ll, 128ll, 129ll, 8192ll, 65537ll, 262144ll, 1ll << 30})
       for (int V : {4, 8}) {
+        // what the launch takes: the plan of the size query and of the other sweeps
         const long long cols = nvec * V;
-        CHECK(p.grid <= rms_bwd_workspace_rows(rows, cols), "partial rows past the workspace");
+        const RmsBwdPlan p = rms_bwd_plan(rows, cols, 16 / V, true, true);
+        CHECK(p.narrow == (nvec > 0 && nvec <= 64), "narrow");
+        if (!p.narrow) continue;
+        const RmsRowPlan& r = p.row;
+        CHECK(r.tpr >= nvec && r.tpr <= 64 && r.kv == 1 && r.rpb * r.tpr == kNarrowBlock && !p.wave, "shape");
+        CHECK(p.grid >= 1 && p.grid <= kBwdGridTarget && p.nparts == p.grid, "grid");
+        CHECK(p.grid * p.steps * r.rpb >= rows, "rows not covered");
+        CHECK((p.grid - 1) * p.steps * r.rpb < rows, "empty workgroup");
+        CHECK(p.nparts <= rms_bwd_workspace_rows(rows, cols), "partial rows past the workspace");
         if (rows <= 129)
           for (long long wg = 0; wg < p.grid; ++wg)
-            for (int sub = 0; sub < p.rpb; ++sub)
+            for (int sub = 0; sub < r.rpb; ++sub)
               for (long long st = 0; st < p.steps; ++st)
-                for (int t = 0; t < p.tpr; ++t) {
-                  const long long off = rms_bwd_load_offset(wg * p.rpb + sub, st, p.grid * p.rpb, p.steps,
-                                                            rows, t, 0, p.tpr, V, nvec, cols);
+                for (int t = 0; t < r.tpr; ++t) {
+                  const long long off = rms_bwd_load_offset(wg * r.rpb + sub, st, p.grid * r.rpb, p.steps,
+                                                            rows, t, 0, r.tpr, V, nvec, cols);
                   CHECK(off >= 0 && off + V <= rows * cols, "load past the matrix");
                 }
       }
-    }
   }
   std::printf("%d failures\n", fails);
   return fails != 0;

@@ -87,9 +87,12 @@ int main() {
                 CHECK(r.block == 64 * kWaveRowsPerBlock && r.rpb == kWaveRowsPerBlock,
                       "wave block shape");
                 CHECK(nvec <= kWaveRowMaxVec, "wave dW staging exceeds its LDS array");
+              } else if (p.narrow) {
+                CHECK(r.kv == 1 && (r.tpr == 8 || r.tpr == 16 || r.tpr == 32 || r.tpr == 64),
+                      "no narrow instantiation for tpr=%d kv=%d", r.tpr, r.kv);
+                CHECK(r.block == kNarrowBlock && r.rpb * r.tpr == kNarrowBlock, "narrow block shape");
               } else {
-                const bool inst = (r.kv == 1 && (r.tpr == 64 || r.tpr == 128 || r.tpr == 256 ||
-                                                  r.tpr == 512)) ||
+                const bool inst = (r.kv == 1 && (r.tpr == 128 || r.tpr == 256 || r.tpr == 512)) ||
                                   (r.tpr == 512 && (r.kv == 2 || r.kv == 4));
                 CHECK(inst, "no bwd instantiation for tpr=%d kv=%d", r.tpr, r.kv);
                 CHECK(r.block == 512 && r.rpb * r.tpr == 512, "bwd block shape");
@@ -100,7 +103,7 @@ int main() {
               CHECK(p.grid * p.steps * r.rpb >= rows, "rows=%lld not covered", rows);
               CHECK(rows == 0 || (p.grid - 1) * p.steps * r.rpb < rows, "empty workgroup");
               CHECK(p.grid < (1ll << 31), "grid too large");
-              if (dw) CHECK(p.nparts == (p.wave ? p.grid : p.grid * r.rpb), "nparts");
+              if (dw) CHECK(p.nparts == (p.wave || p.narrow ? p.grid : p.grid * r.rpb), "nparts");
               // every 16-byte load of the backward kernel lies inside the [rows, ld] matrix
               // (ld = cols and a wider stride), for every workgroup, slot, step and lane
               if (rows > 0 && rows <= 2049 && cols <= 8192) {
@@ -147,7 +150,8 @@ int main() {
         RmsRowPlan f = rms_fwd_plan(nvec);
         if (f.reg) {
           CHECK((long long)f.tpr * f.kv >= nvec, "fwd plan covers %d of %lld", f.tpr * f.kv, nvec);
-          const bool inst = (f.tpr == 64 && (f.kv == 1 || f.kv == 2)) || (f.tpr == 128 && f.kv == 2) ||
+          const bool inst = (f.kv == 1 && (f.tpr == 8 || f.tpr == 16 || f.tpr == 32 || f.tpr == 64)) ||
+                            (f.tpr == 64 && f.kv == 2) || (f.tpr == 128 && f.kv == 2) ||
                             (f.tpr == 256 && f.kv == 2) || (f.tpr == 512 && (f.kv == 2 || f.kv == 4));
           CHECK(inst, "no fwd instantiation for tpr=%d kv=%d", f.tpr, f.kv);
           CHECK(f.block == (f.tpr > 256 ? f.tpr : 256) && f.rpb * f.tpr == f.block, "fwd block shape");
@@ -395,8 +399,12 @@ def test_workspace_query_covers_every_partial_row():
     lib = _lib.load()
     # one partial row per row slot of every backward workgroup: rows small
     # enough that each row group gets its own workgroup
-    for rows, cols in [(37, 8192), (37, 12288), (5, 8192), (129, 12288), (1, 8192), (300, 512)]:
+    for rows, cols in [(37, 8192), (37, 12288), (5, 8192), (129, 12288), (1, 8192)]:
         got = lib.ts_rmsnorm_bwd_workspace_size(rows, cols)
         assert got >= rows * cols * 4 or got >= 512 * cols * 4, (rows, cols, got)
+    # kernels that sum a workgroup's rows write one: 512 fp32 columns a wave a row, four rows a
+    # workgroup; 64 columns of either size at most 64 rows (those of the generic path)
+    assert lib.ts_rmsnorm_bwd_workspace_size(300, 512) == 75 * 512 * 4
+    assert lib.ts_rmsnorm_bwd_workspace_size(4096, 64) == 64 * 64 * 4
     assert lib.ts_rmsnorm_bwd_workspace_size(0, 4096) == 0
     assert lib.ts_rmsnorm_bwd_workspace_size(16, 0) == 0

@@ -22,10 +22,10 @@ constexpr int kWave = 64;
 // ---------------------------------------------------------------------------
 // RMSNorm
 //
-// Register path: a row is owned by `tpr` threads (a power of two, whole
-// waves), each holding `kv` 16-byte vectors spaced tpr vectors apart, so one
-// load instruction of a wave covers 1 KiB of contiguous row. A workgroup holds
-// rpb = block / tpr rows at a time. Few vectors per thread and many small
+// Register path: a row is owned by `tpr` threads (a power of two; whole waves,
+// or 8 to 32 lanes of one where the row is narrow), each holding `kv` 16-byte
+// vectors spaced tpr vectors apart, so one load instruction of a wave covers 1 KiB
+// of contiguous row. A workgroup holds rpb = block / tpr rows at a time. Few vectors per thread and many small
 // workgroups keep the HBM queues full; loops over many vectors per thread do
 // not (measured on MI355X: one 16-byte load per thread copies at ~6.4 TB/s,
 // eight per thread at ~4.2 TB/s).
@@ -33,7 +33,8 @@ constexpr int kWave = 64;
 // Backward: each workgroup walks up to `steps` row groups spaced `grid` apart
 // (grid * steps >= the number of row groups) and keeps the dW contributions
 // of its threads' columns in registers; it writes rpb fp32 partial rows at
-// the end, which a second kernel sums in a fixed order.
+// the end (one where the kernel sums its row slots in LDS first), which a
+// second kernel sums in a fixed order.
 // ---------------------------------------------------------------------------
 constexpr int kMaxKv = 4;                 // vectors per thread on the register path
 // Backward workgroups, 2 per CU on 256 CUs (measured on MI355X at
@@ -46,17 +47,26 @@ inline int vec_elems(int elt_bytes) { return 16 / elt_bytes; }
 
 struct RmsRowPlan {
   bool reg;    // register path possible
-  int tpr;     // threads per row (64..512)
+  int tpr;     // threads per row (8..512)
   int kv;      // vectors per thread (1, 2 or 4)
   int block;   // threads per workgroup
   int rpb;     // rows per workgroup step (block / tpr)
 };
 
-// Forward: two vectors per thread where the row allows it.
+// Narrow rows (the per-head norms: rows of one head of 64 to 256 elements). A row of at most
+// 32 vectors takes 8, 16 or 32 lanes of a wave, so a wave works on 2 to 8 rows at a time
+// where a wave per row would leave up to 7 of 8 lanes idle. 0: not a narrow row.
+inline int rms_narrow_tpr(int64_t nvec) {
+  if (nvec <= 0 || nvec > 32) return 0;
+  return nvec <= 8 ? 8 : nvec <= 16 ? 16 : 32;
+}
+
+// Forward: two vectors per thread where the row allows it, one lane per vector of narrow rows.
 inline RmsRowPlan rms_fwd_plan(int64_t nvec) {
   RmsRowPlan p{false, 0, 0, 0, 0};
   if (nvec <= 0 || nvec > 512 * kMaxKv) return p;
-  if (nvec <= 64) { p.tpr = 64; p.kv = 1; }
+  if (nvec <= 32) { p.tpr = rms_narrow_tpr(nvec); p.kv = 1; }
+  else if (nvec <= 64) { p.tpr = 64; p.kv = 1; }
   else if (nvec <= 128) { p.tpr = 64; p.kv = 2; }
   else if (nvec <= 256) { p.tpr = 128; p.kv = 2; }
   else if (nvec <= 512) { p.tpr = 256; p.kv = 2; }
@@ -68,13 +78,12 @@ inline RmsRowPlan rms_fwd_plan(int64_t nvec) {
   return p;
 }
 
-// Backward: one vector per thread where the row allows it (x and dy are both
-// read, so a thread already has two loads in flight).
+// Backward of rows above 64 vectors: one vector per thread where the row allows it (x and
+// dy are both read, so a thread already has two loads in flight).
 inline RmsRowPlan rms_bwd_row_plan(int64_t nvec) {
   RmsRowPlan p{false, 0, 0, 0, 0};
-  if (nvec <= 0 || nvec > 512 * kMaxKv) return p;
-  if (nvec <= 64) { p.tpr = 64; p.kv = 1; }
-  else if (nvec <= 128) { p.tpr = 128; p.kv = 1; }
+  if (nvec <= 64 || nvec > 512 * kMaxKv) return p;
+  if (nvec <= 128) { p.tpr = 128; p.kv = 1; }
   else if (nvec <= 256) { p.tpr = 256; p.kv = 1; }
   else if (nvec <= 512) { p.tpr = 512; p.kv = 1; }
   else if (nvec <= 1024) { p.tpr = 512; p.kv = 2; }
@@ -109,37 +118,26 @@ inline RmsRowPlan rms_bwd_wave_plan(int64_t nvec) {
   return p;
 }
 
-// Narrow rows (the per-head norms: rows of one head of 64 to 256 elements). A row of at most
-// 32 vectors takes 8, 16 or 32 lanes of a wave, so a wave works on 2 to 8 rows at a time
-// where a wave per row would leave up to 7 of 8 lanes idle. 0: not a narrow row.
-inline int rms_narrow_tpr(int64_t nvec) {
-  if (nvec <= 0 || nvec > 32) return 0;
-  return nvec <= 8 ? 8 : nvec <= 16 ? 16 : 32;
-}
 // Backward of rows of up to 64 vectors (rms_bwd_narrow): kNarrowBlock threads, rpb =
 // kNarrowBlock / tpr rows per step, and one dW partial row per workgroup (its row slots are
 // summed in LDS), at most kBwdGridTarget of them. Measured on MI355X against a wave per row
 // and a partial row per wave at [262144, 128] bf16: 75.7 -> 35.8 us, the sum of the partial
 // rows 21.4 -> 4.1 us (512 of them, not 4096); the forward 60.3 -> 24.3 us.
 constexpr int kNarrowBlock = 1024;
-struct RmsNarrowPlan {
-  int tpr, rpb;
-  int64_t steps, grid;
-};
-inline RmsNarrowPlan rms_bwd_narrow_plan(int64_t rows, int64_t nvec) {
-  RmsNarrowPlan p{0, 0, 0, 0};
+inline RmsRowPlan rms_bwd_narrow_plan(int64_t nvec) {
+  RmsRowPlan p{false, 0, 0, 0, 0};
   if (nvec <= 0 || nvec > 64) return p;
   p.tpr = nvec <= 32 ? rms_narrow_tpr(nvec) : 64;
+  p.kv = 1;
+  p.reg = true;
+  p.block = kNarrowBlock;
   p.rpb = kNarrowBlock / p.tpr;
-  const int64_t groups = (rows + p.rpb - 1) / p.rpb;
-  p.steps = (groups + kBwdGridTarget - 1) / kBwdGridTarget;
-  if (p.steps < 1) p.steps = 1;
-  p.grid = (groups + p.steps - 1) / p.steps;
   return p;
 }
 
 struct RmsBwdPlan {
   bool reg;        // register path (else the generic element-wise kernels)
+  bool narrow;     // register path with up to 64 lanes per row (rms_bwd_narrow)
   bool wave;       // register path with one wave per row (rms_bwd_wave)
   RmsRowPlan row;  // register-path shape
   int64_t steps;   // row groups (of rpb rows) per workgroup
@@ -150,12 +148,14 @@ struct RmsBwdPlan {
 // `vec_ok` says whether pointers and strides allow 16-byte access.
 inline RmsBwdPlan rms_bwd_plan(int64_t rows, int64_t cols, int elt_bytes, bool vec_ok,
                                bool need_dw) {
-  RmsBwdPlan p{false, false, RmsRowPlan{false, 0, 0, 0, 0}, 0, 0, 0};
+  RmsBwdPlan p{false, false, false, RmsRowPlan{false, 0, 0, 0, 0}, 0, 0, 0};
   const int V = vec_elems(elt_bytes);
   if (vec_ok && cols % V == 0) {
-    p.row = rms_bwd_wave_plan(cols / V);
-    p.wave = p.row.reg;
-    if (!p.wave) p.row = rms_bwd_row_plan(cols / V);
+    p.row = rms_bwd_narrow_plan(cols / V);
+    p.narrow = p.row.reg;
+    if (!p.narrow) p.row = rms_bwd_wave_plan(cols / V);
+    p.wave = p.row.reg && !p.narrow;
+    if (!p.row.reg) p.row = rms_bwd_row_plan(cols / V);
   }
   p.reg = p.row.reg;
   if (p.reg) {
@@ -164,8 +164,8 @@ inline RmsBwdPlan rms_bwd_plan(int64_t rows, int64_t cols, int elt_bytes, bool v
     if (steps < 1) steps = 1;
     p.steps = steps;
     p.grid = (groups + steps - 1) / steps;
-    // the wave kernel sums its rows' dW in LDS: one partial row per workgroup
-    p.nparts = need_dw ? (p.wave ? p.grid : p.grid * p.row.rpb) : 0;
+    // the narrow and wave kernels sum their rows' dW in LDS: one partial row per workgroup
+    p.nparts = need_dw ? (p.narrow || p.wave ? p.grid : p.grid * p.row.rpb) : 0;
   } else {
     p.steps = 0;
     p.grid = rows;

@@ -1,8 +1,8 @@
 // RMSNorm forward/backward for gfx950.
 //
 // Register path (ts_plan::rms_fwd_plan / rms_bwd_row_plan): a row is owned by
-// TPR threads (whole waves), each holding KV 16-byte vectors spaced TPR
-// vectors apart, so every load instruction of a wave covers 1 KiB of
+// TPR threads (whole waves, or 8 to 32 lanes of one for rows of up to 32
+// vectors), each holding KV 16-byte vectors spaced TPR vectors apart, so every load instruction of a wave covers 1 KiB of
 // contiguous row and each thread has only one or two loads in flight per
 // tensor; the row stays in VGPRs between the reduction and the output, so x
 // (and dy) are read from HBM exactly once. The sum of squares (forward) and
@@ -789,11 +789,7 @@ ts_status fwd_typed(const void* x, int64_t ldx, const void* w, void* y, int64_t 
   const W* wp = static_cast<const W*>(w);
   T* yp = static_cast<T*>(y);
   const int64_t nvec = cols / V;
-  ts_plan::RmsRowPlan plan = ts_plan::rms_fwd_plan(nvec);
-  if (const int tpr = ts_plan::rms_narrow_tpr(nvec)) {
-    plan.tpr = tpr;
-    plan.rpb = plan.block / tpr;
-  }
+  const ts_plan::RmsRowPlan plan = ts_plan::rms_fwd_plan(nvec);
   const bool add_ok = !kAdd || (vec_ok<T, W>(add.r, add.ldr, cols, nullptr) &&
                                 (add.h == nullptr || vec_ok<T, W>(add.h, add.ldh, cols, nullptr)));
   if (vec_ok<T, W>(x, ldx, cols, w) && vec_ok<T, W>(y, ldy, cols, nullptr) && add_ok &&
@@ -839,22 +835,19 @@ ts_status bwd_typed(const void* dy, int64_t lddy, const void* x, int64_t ldx, co
   const int64_t nvec = cols / V;
   const bool vec = vec_ok<T, W>(x, ldx, cols, w) && vec_ok<T, W>(dy, lddy, cols, nullptr) &&
                    vec_ok<T, W>(dx, lddx, cols, nullptr);
-  ts_plan::RmsBwdPlan plan =
+  const ts_plan::RmsBwdPlan plan =
       ts_plan::rms_bwd_plan(rows, cols, (int)sizeof(T), vec, dw != nullptr);
-  const ts_plan::RmsNarrowPlan narrow =
-      ts_plan::rms_bwd_narrow_plan(rows, plan.reg ? nvec : 0);
-  if (narrow.tpr != 0) plan.nparts = dw != nullptr ? narrow.grid : 0;
   if (dw != nullptr && (size_t)plan.nparts * (size_t)cols * sizeof(float) > ws_bytes)
     return ts_host::fail(TS_ERR_WORKSPACE, "rmsnorm_bwd: plan needs %lld partial rows",
                          (long long)plan.nparts);
-  if (narrow.tpr != 0) {
+  if (plan.narrow) {
     float* part = dw != nullptr ? ws : nullptr;
     bool launched = false;
 #define TS_LAUNCH_NARROW(TPR)                                                                  \
-  if (narrow.tpr == TPR) {                                                                     \
-    hipLaunchKernelGGL((rms_bwd_narrow<T, W, TPR>), dim3((unsigned)narrow.grid),               \
+  if (plan.row.tpr == TPR) {                                                                   \
+    hipLaunchKernelGGL((rms_bwd_narrow<T, W, TPR>), dim3((unsigned)plan.grid),                 \
                        dim3(ts_plan::kNarrowBlock), 0, st, dyp, lddy, xp, ldx, wp, rstd, dxp,  \
-                       lddx, part, rows, narrow.steps, (int)nvec, (float)cols);                \
+                       lddx, part, rows, plan.steps, (int)nvec, (float)cols);                  \
     launched = true;                                                                           \
   }
     TS_LAUNCH_NARROW(8)
@@ -864,7 +857,7 @@ ts_status bwd_typed(const void* dy, int64_t lddy, const void* x, int64_t ldx, co
 #undef TS_LAUNCH_NARROW
     if (!launched)
       return ts_host::fail(TS_ERR_INVALID_ARGUMENT, "rmsnorm_bwd: bad narrow plan (tpr=%d)",
-                           narrow.tpr);
+                           plan.row.tpr);
     ts_status s = ts_host::check_launch("rms_bwd_narrow");
     if (s != TS_OK) return s;
   } else if (plan.wave) {
