@@ -50,6 +50,16 @@ int main() {
         for (long long last : {1ll, K / 3 + 1, K})
           CHECK(k.splits * split_kper(last, k.splits) >= last, "last chunk");
       }
+  // the bound is met by some H, and a few rows do not ask for what a full tile of them would
+  for (long long M : {1, 8, 256, 300, 2048, 32768}) {
+    long long most = 0;
+    for (long long ht = 1; ht <= 256; ++ht) {
+      const long long b = hidden_split_bytes(M, ht * 256, 1ll << 40);
+      most = b > most ? b : most;
+    }
+    CHECK(most == hidden_split_bytes_any_shape(M), "bound of %lld rows: %lld, needed %lld", M,
+          (long long)hidden_split_bytes_any_shape(M), most);
+  }
   // a tile for every CU: one slot
   CHECK(hidden_split(4096, 4096, 128256).splits == 1, "C5 chunk is not split");
   CHECK(hidden_split(1024, 768, 50257).splits == 21, "12 tiles");

@@ -348,13 +348,15 @@ inline KSplit hidden_split(int64_t M, int64_t H, int64_t K) {
   return KSplit{s, split_kper(K, s)};
 }
 // Bytes of the fp32 partials of one such GEMM ([splits][M][H]), and a bound on them for
-// any H where a workspace query does not know it (at most one tile per CU when split).
+// any H where a workspace query does not know it: the pieces are at most one per CU, so
+// splits * ceil(H / 256) is at most kCus / ceil(M / 256).
 inline int64_t hidden_split_bytes(int64_t M, int64_t H, int64_t K) {
   const KSplit k = hidden_split(M, H, K);
   return k.splits > 1 ? k.splits * M * H * 4 : 0;
 }
 inline int64_t hidden_split_bytes_any_h(int64_t M, int64_t K) {
-  return hidden_split(M, 1, K).splits > 1 ? kCus * kGemmTile * kGemmTile * 4 : 0;
+  const int64_t row_tiles = (M + kGemmTile - 1) / kGemmTile;
+  return hidden_split(M, 1, K).splits > 1 ? kCus / row_tiles * M * kGemmTile * 4 : 0;
 }
 inline int64_t hidden_split_bytes_any_shape(int64_t M) {
   return hidden_split_bytes_any_h(M, (int64_t)1 << 40);
