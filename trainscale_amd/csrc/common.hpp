@@ -229,6 +229,23 @@ constexpr float kLn2 = 0.6931471805599453f;
 
 __device__ inline float fast_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// exp(z - m) formed as exp2(fma(z, log2 e, -m log2 e)) carries the rounding of m log2 e, up to
+// 2^-24 |m| log2 e in the exponent: below this magnitude at most 0.07, past it as much as the
+// sum's whole range, and the product overflows where logits are masked with their type's
+// lowest value (-3.4e38 in bf16 and fp32). References at or past it take sum_exp_far.
+constexpr float kRefMax = 0x1p20f;
+
+// Sum of exp(z - m) over a vector for any reference m that is no less than its values. m is
+// -inf only while every value seen is -inf, whose terms are 0, or NaN.
+template <int VE>
+__device__ inline float sum_exp_far(const float (&z)[VE], float m) {
+  const float ref = m == -INFINITY ? 0.f : m;
+  float cs = fast_exp2((z[0] - ref) * kLog2e);
+#pragma unroll
+  for (int i = 1; i < VE; ++i) cs += fast_exp2((z[i] - ref) * kLog2e);
+  return cs;
+}
+
 }  // namespace ts
 
 // ---------------------------------------------------------------------------

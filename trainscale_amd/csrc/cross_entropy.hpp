@@ -203,23 +203,6 @@ __device__ inline int64_t tail_col(int64_t V) {
   return ts_plan::tail_col(V, (int)threadIdx.x, VE);
 }
 
-// exp(z - m) formed as exp2(fma(z, log2 e, -m log2 e)) carries the rounding of m log2 e, up to
-// 2^-24 |m| log2 e in the exponent: below this magnitude at most 0.07, past it as much as the
-// sum's whole range, and the product overflows where logits are masked with their type's
-// lowest value (-3.4e38 in bf16 and fp32). References at or past it take sum_exp_far.
-constexpr float kRefMax = 0x1p20f;
-
-// Sum of exp(z - m) over a vector for any reference m that is no less than its values. m is
-// -inf only while every value seen is -inf, whose terms are 0, or NaN.
-template <int VE>
-__device__ inline float sum_exp_far(const float (&z)[VE], float m) {
-  const float ref = m == -INFINITY ? 0.f : m;
-  float cs = fast_exp2((z[0] - ref) * kLog2e);
-#pragma unroll
-  for (int i = 1; i < VE; ++i) cs += fast_exp2((z[i] - ref) * kLog2e);
-  return cs;
-}
-
 // Adds the value z to an online (max, sum of exp) pair; nothing for -inf.
 __device__ inline void fold1(float z, float& m, float& s) {
   const float mn = __builtin_fmaxf(m, z);

@@ -14,11 +14,13 @@
 //
 // Stats: one row per workgroup, held in registers (kKv 16-byte vectors per
 // thread). Each lane sums exp(z - m) against one reference, the largest value
-// of its first vector, and folds again with an exact online max only when the
-// sum ends outside [0.5, inf) (extreme logits); then wave and workgroup
-// combine the lanes' (m, s) pairs. Merge: one thread per row, one online
-// pass over the P partials. Backward: one-shot grid over (row, chunk of 256
-// vectors), one vector per thread.
+// of its first vector, and folds again with an exact online max only when the sum
+// ends outside [0.5, 2^60] (extreme logits); then wave and workgroup combine the
+// lanes' (m, s) pairs. Below 2^60 the lanes' sums together stay finite, and a lane
+// whose reference lies so far below another's that its factor flushes to zero held
+// less than 2^60 2^-126, nothing beside the other's 0.5. Merge: one thread per row,
+// one online pass over the P partials. Backward: one-shot grid over (row, chunk of
+// 256 vectors), one vector per thread.
 #include <math.h>
 
 #include "common.hpp"
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(kBlock) void shard_stats_vec(const T* __restrict__ 
     if ((k + 1) * kBlock <= nvec) fold(buf[k], k == 0);
     else if ((int)threadIdx.x + k * kBlock < nvec) fold(buf[k], k == 0);
   }
-  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s < INFINITY)) {
+  if ((int)threadIdx.x < nvec && !(s >= 0.5f && s <= 0x1p60f && fabsf(m) < kRefMax)) {
     // Extreme logits: fold again with an exact online max.
     m = -INFINITY;
     s = 0.f;
@@ -128,11 +130,10 @@ __global__ __launch_bounds__(kBlock) void shard_stats_vec(const T* __restrict__ 
       if ((int)threadIdx.x + k * kBlock < nvec) {
         float z[VE];
         Elt<T>::unpack(buf[k], z);
+        // __builtin_fmaxf drops NaN, whose term makes s NaN, and s stays so
         const float mn = __builtin_fmaxf(m, vmax(z));
-        if (mn != -INFINITY) {
-          s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) + sum_exp(z, mn * kLog2e);
-          m = mn;
-        }
+        s = (s == 0.f ? 0.f : s * fast_exp2((m - mn) * kLog2e)) + sum_exp_far<VE>(z, mn);
+        m = mn;
       }
     }
   }
@@ -199,7 +200,8 @@ __global__ __launch_bounds__(kMergeThreads) void shard_merge(
       if (p0 + u == self) sz = st[u].sum_z;
     }
   }
-  const float lse = gm == -INFINITY ? -INFINITY : gm + logf(gs);
+  // gs is NaN where a rank's partial is, gm still -inf if no other rank has a value
+  const float lse = gm == -INFINITY && gs == 0.f ? -INFINITY : gm + logf(gs);
   float loss = lse - zt;
   if (smoothing != 0.f) loss = (1.f - smoothing) * loss + smoothing * (lse - sz * inv_vp);
   lse_out[row] = lse;
