@@ -271,8 +271,8 @@ ts_status ts_ce_bwd(const void* logits, int64_t ld, ts_dtype dtype,
  * ignore_index (at least 1), 1 sum, 2 mean over all rows (at least 1).
  * ts_ce_loss_weight: *weight = d(reduced loss)/d(row loss) * (hint ? *hint : 1),
  *   the one-element dloss of ts_ce_fwd_bwd; *used (optional) = the hint factor.
- * ts_ce_reduce_loss: *loss = the reduced loss of loss_rows [N] (summed in
- *   double, divided in fp32).
+ * ts_ce_reduce_loss: *loss = the reduced loss of loss_rows [N] (summed and
+ *   divided in double, rounded once).
  * labels: int64 [N]; read for reduction 0 only. All results are fp32 device
  * scalars; N = 0 gives loss 0. Replaces the reduction and the scale of
  * FusedCrossEntropyFunction (loss/sota_losses.py:437-532).

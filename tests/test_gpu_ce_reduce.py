@@ -1,6 +1,6 @@
 """The row weight and the reduced loss formed by one workgroup, at the sizes where its loop
-and the switch to torch's reductions turn, against float64: a double sum rounded to fp32 and
-divided in fp32 is within two fp32 roundings of the exact value."""
+and the switch to torch's reductions turn, against float64. The weight is one fp32 division, the
+loss a double sum divided in double and rounded once: half an fp32 ulp each."""
 import pytest
 import torch
 

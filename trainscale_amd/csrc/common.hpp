@@ -167,9 +167,11 @@ __device__ inline void buf_st16_stream(const u32x4& v, Rsrc r, int voff) {
 // with the row's result), then the four row results are read with
 // v_readlane_b32 and combined in a fixed order. Every lane gets the result.
 //
-// The gfx950 v_permlane16_swap/v_permlane32_swap builtins are not used: with
-// the same value passed as both operands, hipcc (ROCm 7.2) keeps only the
-// first of the two results, which turns the cross-row sum into a doubling.
+// linear_ce.hip combines rows with v_permlane16_swap, the same value as both
+// operands (the compiler copies the register first). The elements of the vector
+// that builtin returns must be copied to scalars before a __builtin_bit_cast:
+// hipcc (ROCm 7.2) reads element 0 for either in the cast of an element, which
+// turns the cross-row sum into a doubling.
 // ---------------------------------------------------------------------------
 
 template <int kCtrl>

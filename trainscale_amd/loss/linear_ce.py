@@ -1,4 +1,4 @@
-"""Fused linear cross-entropy: loss of (hidden @ weight.T) without materialising the logits.
+"""Fused linear cross-entropy: loss of (hidden @ weight.T), the logits formed in bounded chunks.
 
 TrainScale has no such op; its nearest relative is
 ``chunked_log_softmax(hidden, lm_head[V, H], input_ids)`` (rl_training.py:138-191),
@@ -12,17 +12,18 @@ Two schedules run on the gfx950 kernels:
   forward (``ts_flce_forward``) runs the logits GEMM once and keeps only
   per-row softmax statistics and the label's logit; no logits are stored. The
   backward (``ts_flce_backward``) recomputes the logits one vocabulary chunk
-  at a time (about V/8 columns), forms the chunk's dlogits in the GEMM's
-  epilogue and runs the two gradient GEMMs on them: grad_hidden accumulates
-  over the chunks in fp32, grad_weight's rows of the chunk are written
-  directly. Scratch: N x chunk bf16 dlogits plus N x H fp32.
+  at a time (about V/8 columns, or as many as keep the chunk's dlogits at
+  256 MB), forms the chunk's dlogits in the GEMM's epilogue and runs the two
+  gradient GEMMs on them: grad_hidden accumulates over the chunks in fp32,
+  grad_weight's rows of the chunk are written directly. Scratch: N x chunk bf16
+  dlogits plus N x H fp32, or one such sum for each K slot.
 * ``"fused"`` (mean/sum, no transforms): one call (``ts_flce_fwd_bwd``) forms
   the loss and both gradients for an upstream gradient of 1, token chunk by
-  token chunk: half the tokens by default, whose bf16 logits are the only
-  [rows, V] scratch (half the [N, V] logits), with grad_weight summed over the
-  chunks in its bf16 output (one bf16 rounding of the partial sum between the
-  chunks; fp32 accumulation is opt-in); the backward scales the gradients in
-  place. Three GEMMs instead of four.
+  token chunk: by default all the tokens while their bf16 logits fit in 1 GiB,
+  else half of them. The chunk's logits are the only [rows, V] scratch; with two
+  chunks grad_weight is summed in its bf16 output (one bf16 rounding of the
+  partial sum between them; fp32 accumulation is opt-in). The backward scales
+  the gradients in place. Three GEMMs instead of four.
 * ``"stored_logits"`` (opt-in; any reduction and transform): the two-pass
   forward also keeps the bf16 logits ([N, V], N * V * 2 bytes, as the
   reference's chunked_log_softmax keeps each chunk's logits for autograd);
@@ -492,7 +493,7 @@ def fused_linear_cross_entropy(hidden: Tensor, weight: Tensor, labels: Tensor,
                                vocab_chunk: Optional[int] = None,
                                chunk_tokens: Optional[int] = None,
                                grad_weight_accum: str = "bf16") -> Tensor:
-    """Cross-entropy of hidden @ weight.T against labels, without all logits in memory.
+    """Cross-entropy of hidden @ weight.T against labels, with the logits in bounded chunks.
 
     hidden [..., H] and weight [V, H] in bfloat16 (the lm_head layout of
     rl_training.py:156-162); labels [...] int64, ignore_index rows skipped.
@@ -503,12 +504,14 @@ def fused_linear_cross_entropy(hidden: Tensor, weight: Tensor, labels: Tensor,
     (per-row losses, shaped like labels).
 
     schedule: "auto" (default), "fused", "two_pass" or "stored_logits" (module
-    docstring). "fused": chunk_tokens rows per token chunk (None: half of
-    the tokens, 0: one chunk, i.e. all [N, V] logits), grad_weight_accum "bf16"
-    (summed in the bf16 output) or "fp32" (a V x H fp32 workspace); a second
-    backward through its graph raises. "two_pass": vocab_chunk columns per
-    recomputed chunk (None: about V/8). "stored_logits": the two-pass schedule
-    with the bf16 logits kept from the forward to the backward (N * V * 2 bytes).
+    docstring). "fused": chunk_tokens rows per token chunk (None: all the tokens
+    while their bf16 logits fit in 1 GiB, else half of them; 0: one chunk, i.e. all
+    [N, V] logits), grad_weight_accum "bf16" (summed in the bf16 output) or "fp32"
+    (a V x H fp32 workspace); a second backward through its graph raises.
+    "two_pass": vocab_chunk columns per recomputed chunk (None: about V/8, or as
+    many as keep the chunk's dlogits at 256 MB). "stored_logits": the two-pass
+    schedule with the bf16 logits kept from the forward to the backward (N * V * 2
+    bytes).
     """
     if schedule == "auto":
         grads = torch.is_grad_enabled() and (hidden.requires_grad or weight.requires_grad)
