@@ -405,14 +405,15 @@ void rms_bwd_narrow(const T* __restrict__ dy, int64_t lddy, const T* __restrict_
     if (ok) {
       float o[V];
 #pragma unroll
-      for (int i = 0; i < V; ++i) o[i] = rstd * (df[i] * wf[i] - (xf[i] * rstd) * c1);
+      for (int i = 0; i < V; ++i)  // dy * w unrounded, as s's product is not
+        o[i] = rstd * __builtin_fmaf(df[i], wf[i], -((xf[i] * rstd) * c1));
       st16_stream(dx + row * lddx + (int64_t)t * V, Elt<T>::pack(o));
     }
   }
 
   if (partial == nullptr) return;  // dW not requested
-  // row slots [kRpb][nq quads], summed by groups of nq threads: group g takes the slots
-  // g, g + groups, ..., then the first nq threads the groups' sums
+  // row slots [kRpb][nq quads], summed by halves: a sum in one chain over the slots lost up to
+  // twice as much ([64, 64] fp32 dW 1.7e-7 against 8.9e-8) and took longer
   const int nq = nvec * V / 4;
   if (in_row) {
 #pragma unroll
@@ -420,34 +421,22 @@ void rms_bwd_narrow(const T* __restrict__ dy, int64_t lddy, const T* __restrict_
       dw_lds[sub * nq + t * (V / 4) + h] =
           make_float4(acc[4 * h], acc[4 * h + 1], acc[4 * h + 2], acc[4 * h + 3]);
   }
-  __syncthreads();
-  const int groups = kBlock / nq < kRpb ? kBlock / nq : kRpb;
-  const int g = threadIdx.x / nq;
-  const int q = threadIdx.x - g * nq;
-  float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (g < groups) {
-    for (int j = g; j < kRpb; j += groups) {
-      const float4 u = dw_lds[j * nq + q];
+  static_assert(V <= 8, "the lower half's quads, TPR * V / 4 * kRpb / 2, within the threads");
+  const int tid = threadIdx.x;
+  for (int n = kRpb / 2 * nq; n >= nq; n >>= 1) {  // quads of the lower half
+    __syncthreads();
+    if (tid < n) {
+      float4 a = dw_lds[tid];
+      const float4 u = dw_lds[tid + n];
       a.x += u.x;
       a.y += u.y;
       a.z += u.z;
       a.w += u.w;
+      dw_lds[tid] = a;
     }
   }
-  __syncthreads();
-  if (g < groups) dw_lds[g * nq + q] = a;
-  __syncthreads();
-  if ((int)threadIdx.x < nq) {
-    float4 b = dw_lds[threadIdx.x];
-    for (int j = 1; j < groups; ++j) {
-      const float4 u = dw_lds[j * nq + threadIdx.x];
-      b.x += u.x;
-      b.y += u.y;
-      b.z += u.z;
-      b.w += u.w;
-    }
-    reinterpret_cast<float4*>(partial + (int64_t)blockIdx.x * nvec * V)[threadIdx.x] = b;
-  }
+  if (tid < nq)  // thread tid wrote that quad itself
+    reinterpret_cast<float4*>(partial + (int64_t)blockIdx.x * nvec * V)[tid] = dw_lds[tid];
 }
 
 // ---------------------------------------------------------------------------
