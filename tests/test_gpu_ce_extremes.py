@@ -127,3 +127,19 @@ def test_lse_does_not_depend_on_the_reference(gpu, V, low):
         ulp = 2.0 ** (ref.log2().floor() - 23)
         err = (lse.double() - ref) / ulp
         assert err.pow(2).mean().sqrt().item() <= 0.9, (lead, err.pow(2).mean().sqrt().item())
+
+
+@pytest.mark.parametrize("V", [1000, 1001, 4003])
+@pytest.mark.parametrize("off", [160.0, -1000.0])
+def test_lse_of_offset_logits(gpu, V, off):
+    """With logits far from 0 on one side the sum's errors lie below an ulp of lse: what is left is
+    its own rounding, sqrt(1 / 12) = 0.2887 ulp rms, and no bias, in both schedules."""
+    g = torch.Generator(device=gpu).manual_seed(V)
+    x = 2 * torch.randn(8192, V, generator=g, device=gpu) + off
+    labels = torch.zeros(8192, dtype=torch.long, device=gpu)
+    ref = x.double().logsumexp(1)
+    ulp = 2.0 ** (ref.abs().log2().floor() - 23)
+    one = torch.ones(1, device=gpu)
+    for lse in (ops.ce_forward_backward(x, V, labels, one)[1], ops.ce_forward(x, V, labels)[1]):
+        err = (lse.double() - ref) / ulp
+        assert err.pow(2).mean().sqrt() <= 0.297 and err.mean().abs() <= 0.02

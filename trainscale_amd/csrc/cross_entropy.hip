@@ -119,10 +119,12 @@ __global__ __launch_bounds__(kThreads) void ce_fwd_vec(const T* __restrict__ log
     }
     if (fabsf(m) < kRefMax) {
       const float mb = m * kLog2e;
+      float cs = 0.f;
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u)
 #pragma unroll
-        for (int i = 0; i < VE; ++i) s += fast_exp2(__builtin_fmaf(z[u][i], kLog2e, -mb));
+        for (int i = 0; i < VE; ++i) cs += fast_exp2(__builtin_fmaf(z[u][i], kLog2e, -mb));
+      s += __builtin_fmaf(cs, -bias_lack(m, mb), cs);
     } else {
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) s += sum_exp_far<VE>(z[u], m);
@@ -146,8 +148,10 @@ __global__ __launch_bounds__(kThreads) void ce_fwd_vec(const T* __restrict__ log
     }
     if (fabsf(m) < kRefMax) {
       const float mb = m * kLog2e;
+      float cs = 0.f;
 #pragma unroll
-      for (int i = 0; i < VE; ++i) s += fast_exp2(__builtin_fmaf(z[i], kLog2e, -mb));
+      for (int i = 0; i < VE; ++i) cs += fast_exp2(__builtin_fmaf(z[i], kLog2e, -mb));
+      s += __builtin_fmaf(cs, -bias_lack(m, mb), cs);
     } else {
       s += sum_exp_far<VE>(z, m);
     }
