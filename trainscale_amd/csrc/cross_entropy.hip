@@ -163,7 +163,7 @@ __global__ __launch_bounds__(kThreads) void ce_fwd_vec(const T* __restrict__ log
   }
   block_fold(m, s, sz, lds);
   if (threadIdx.x == 0) {
-    const float l = m + logf(s);
+    const float l = log_sum(m, s);
     loss[row] = row_loss<kMode>(xr, label, V, ignore_index, l, sz, smoothing, xf);
     lse_out[row] = l;
   }

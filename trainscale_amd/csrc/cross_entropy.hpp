@@ -253,21 +253,39 @@ __device__ inline float bias_lack(float m, float mb) {
   return kLn2 * __builtin_fmaf(m, kLog2e, -mb);
 }
 
+constexpr float kLn2Lo = (float)(0.6931471805599453 - (double)kLn2);
+
+// m + log(s), rounded about once: the exponent of s joins m, what that sum loses the logarithm
+// of the rest. m + logf(s) adds logf's rounding, half an ulp of up to 7 in an lse of 8 or more.
+__device__ inline float log_sum(float m, float s) {
+  const int e = __builtin_amdgcn_frexp_expf(s) - 1;
+  const float k = (float)e;
+  const float y = __builtin_amdgcn_logf(__builtin_amdgcn_ldexpf(s, -e));  // v_log_f32: log2
+  const float a = __builtin_fmaf(k, kLn2, m);
+  const float b = __builtin_fmaf(k, kLn2, m - a);
+  const float l = a + __builtin_fmaf(y, kLn2, __builtin_fmaf(k, kLn2Lo, b));
+  return s == 0.f ? -INFINITY : l;  // nothing but -inf in the row
+}
+
 // Moves a lane's (m, sum of exp2(z log2 e - mb)) pair, mb = m log2 e rounded, to a reference
-// next to its sum: s about in [0.5, 1) and m + log(s) the lane's log-sum, without the roundings
+// next to its sum: s about in [1, 2) and m + log(s) the lane's log-sum, without the roundings
 // of mb and of log2 e and, where m lay far below the lane's values, without two large terms
-// that cancel. What the new m lost in its rounding goes into s.
-// Rms error of lse at [512, 1001] fp32 N(0, 1), the first 256 columns 20 lower: 1.46 ulp
-// without, 0.62 now; for rows that do not begin so 0.64 and 0.52.
+// that cancel. What the new m lost in its rounding goes into s. Rms error of lse at [512, 1001]
+// fp32 N(0, 1), with log_sum: 0.31 ulp, 0.30 to 0.38 with the first 256 columns 10 to 40 lower;
+// without either 0.64 and 1.1 to 2.6.
 __device__ inline void settle(float& m, float mb, float& s) {
-  // of k ln 2, in the units of m, ln 2's rounding, and of the terms' exponents, whose values lie
-  // about k ln 2 above m, the rounding of log2 e
+  // ln 2 in 15 bits, so that a whole multiple of it is exact, and so is its sum with a larger m of
+  // the other sign; the rest of ln 2 goes into s, with the rounding of log2 e over the distance
+  // that the terms lie above m
+  constexpr float kHi = 0.693145751953125f;
   constexpr double kL = 0.6931471805599453, kE = 1.4426950408889634;
-  constexpr float kLo = (float)(kL - (double)kLn2 + kL * kL * (kE - (double)kLog2e));
-  const float k = (float)__builtin_amdgcn_frexp_expf(s);
-  const float m1 = __builtin_fmaf(k, kLn2, m);
-  const float lost = __builtin_fmaf(k, kLn2, m - m1) + __builtin_fmaf(k, kLo, -bias_lack(m, mb));
-  const float s1 = __builtin_amdgcn_frexp_mantf(s);
+  constexpr float kRest = (float)(kL - (double)kHi + kL * kL * (kE - (double)kLog2e));
+  const int e = __builtin_amdgcn_frexp_expf(s) - 1;
+  const float k = (float)e;
+  const float d = k * kHi;
+  const float m1 = m + d;
+  const float lost = __builtin_fmaf(k, kRest, ((m - m1) + d) - bias_lack(m, mb));
+  const float s1 = __builtin_amdgcn_ldexpf(s, -e);
   s = __builtin_fmaf(s1, lost, s1);
   m = m1;
 }
@@ -298,7 +316,7 @@ __device__ inline float fused_lse(float m, float s, float& sz, float* lds) {
     if constexpr (kMode != kPlain) gz += lds[2 * kNW + i];
   }
   if constexpr (kMode != kPlain) sz = gz;
-  return gm + logf(gs);
+  return log_sum(gm, gs);
 }
 
 template <typename G>
@@ -310,21 +328,11 @@ constexpr uint32_t sign_bits() {
 // six at 8 and eight at 4.
 constexpr int fused_waves(int kv) { return kv >= 16 ? 4 : kv >= 8 ? 6 : 8; }
 
-// Largest sum of exp(z - m) that a lane's reference m serves for (see ce_fused_vec). The lower
-// the bound, the nearer the exponents of the terms that matter are to 0, where they are rounded
-// finest; but a wave with a lane that holds a logit log(bound) above its first vector folds its
-// vectors twice. With 2^20 lse errors do not depend on where the first vectors lie; with 2^40
-// and 2^60 they grow from 0.6 to 0.7 and 0.9 ulp rms where these lie 20 and 30 below the row.
-// 2^20 is for the rows that older kernels folded with an exact online max (short ones and
-// those off 16-byte boundaries; measured on MI355X, [4096, 50257] bf16 of N(0, 4): 191 against
-// 189 us with 2^60). Aligned longer rows had no such fold: [8192, 128256] with 64 logits a row
-// 22 high takes 796 us with 2^16, 732 with 2^60. With transforms a second fold costs most
-// ([4096, 50257], softcap 30, N(0, 6): 297 us with 2^20, 253 with 2^40), and the rounding of the
-// transformed logits themselves covers the difference.
-template <int kMode, int kThr, int kKv, bool kAligned>
-constexpr float lane_sum_max() {
-  return kAligned && kThr * kKv > 1024 ? 0x1p60f : kMode == kGeneral ? 0x1p40f : 0x1p20f;
-}
+// Largest sum of exp(z - m) that a lane's reference m serves for (see ce_fused_vec): one whose
+// terms' exponents, up to 60, are still rounded finely beside lse. A lower bound costs more
+// second folds (2^20: [4096, 50257] bf16 of N(0, 6), softcap 30, 297 us instead of 253) and
+// gains nothing: with settle, lse errors do not depend on where the first vectors lie.
+constexpr float kLaneSumMax = 0x1p60f;
 
 template <typename T, typename G, int kMode, int kThr, int kKv, bool kAligned>
 __global__ __launch_bounds__(kThr) __attribute__((amdgpu_waves_per_eu(fused_waves(kKv))))
@@ -335,7 +343,6 @@ void ce_fused_vec(
     G* __restrict__ grad, int64_t ld_grad) {
   constexpr int VE = Elt<T>::kVec;
   constexpr int kNW = kThr / kWave;
-  constexpr float kLaneSumMax = lane_sum_max<kMode, kThr, kKv, kAligned>();
   constexpr int kGradBytes = VE * (int)sizeof(G);  // grad bytes per logits vector
   __shared__ float lds[3 * kNW];
   const int64_t row = blockIdx.x;
@@ -412,7 +419,7 @@ void ce_fused_vec(
   // Each lane sums exp(z - m) over its vectors against one reference m, the
   // largest value of its first vector (0 if that vector is all -inf): per
   // element one unpack, one FMA, one exp and one add, with no running max or
-  // rescale. Such a sum serves while it lies in [0.5, lane_sum_max]: terms that
+  // rescale. Such a sum serves while it lies in [0.5, kLaneSumMax]: terms that
   // underflowed are then below its resolution, and settle brings it next to its
   // reference, so that no fold over the lanes overflows with it or loses it.
   // Other lanes (values far above m, a NaN, a reference past kRefMax, an all -inf
